@@ -1075,6 +1075,18 @@ void nova_weight_grad(nova_handle_t h, const void* d_input, const void* d_grad_o
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
         cus < 1)
         cus = 256;
+    if (!grad_f32) {
+        const WgradDirectPlan dp = wgrad_direct_plan(batch, C, K, H, W, pad, cus);
+        if (dp.ok) {
+            if (dp.ws_bytes > 0 && !ensure_ws(Hd, (size_t)dp.ws_bytes)) return;
+            hip_ok(launch_wgrad_direct(static_cast<const uint16_t*>(d_input),
+                                       static_cast<const uint16_t*>(d_grad_output),
+                                       static_cast<float*>(d_grad_weight), batch, C, K, H, W, pad,
+                                       dp, Hd->ws, Hd->stream),
+                   "weight gradient");
+            return;
+        }
+    }
     const WgradPlan pl = wgrad_plan(batch, C, K, H, W, pad, cus);
     if (!pl.ok) {
         set_error(kErrInvalidArgument,

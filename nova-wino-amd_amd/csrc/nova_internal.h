@@ -301,4 +301,21 @@ hipError_t launch_wgrad(const uint16_t* x, const void* dy, bool dy_f32, float* d
                         int K, int H, int W, int pad, const WgradPlan& plan, void* ws,
                         hipStream_t s);
 
+// Direct form for fp16 dY (wgrad_direct.hip): nine taps as fp16 MFMA products
+// over the pixels, the operands read as they are, fp32 sums. ok is false
+// where the form does not apply (pads above 2, no images, images of 1 GiB).
+struct WgradDirectPlan {
+    int wk, wc;         // waves along output and input channels (of 8)
+    int G, R, nrb;      // images and x rows per unit, row blocks per image
+    int Ws, nstrip;     // 8-pixel segments per column strip, strips per row
+    int lo, XS, XP, xpitch, dpitch, dstart, zero, nblk, nwx;  // LDS geometry (16-byte chunks)
+    int ntk, nt, nunits, nsplit;
+    int64_t ws_bytes;   // the splits' partial filters (none with one split)
+    bool ok;
+};
+WgradDirectPlan wgrad_direct_plan(int B, int C, int K, int H, int W, int pad, int cus);
+hipError_t launch_wgrad_direct(const uint16_t* x, const uint16_t* dy, float* dw, int B, int C,
+                               int K, int H, int W, int pad, const WgradDirectPlan& plan,
+                               void* ws, hipStream_t s);
+
 }  // namespace nova

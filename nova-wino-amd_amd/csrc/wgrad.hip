@@ -1,4 +1,6 @@
-// Weight gradient of the NOVA F(6,3) convolution, on the Winograd domain.
+// Weight gradient of the NOVA F(6,3) convolution, on the Winograd domain:
+// float32 output gradients, pads above 2 and tensors of 2 GiB and more (the
+// rest runs as direct float16 products, wgrad_direct.hip).
 //
 // The reference's backward computes dL/dw in fp32 PyTorch with a per-sample
 // unfold loop (/root/reference/nova_winograd/conv2d.py:121-147). Here it is

@@ -1,0 +1,109 @@
+"""The direct weight gradient (fp16 output gradients, nova_weight_grad) at the
+edges of its units: odd widths (staged through registers), widths off the
+8-pixel chunk (masked), whole chunks, several images per unit, column strips,
+pads 0 to 2, channels off the 32-blocks, and both tensors off every 4-byte
+address.
+
+Bound: the products of fp16 values are exact, so each entry's error is that of
+an fp32 sum of n = B*Ho*Wo terms, at most n * 2^-23 * sum |dY||x| (one unit in
+the last place per addition, whichever way the matrix unit rounds).
+"""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = torch.device("cuda:0")
+
+# (B, C, K, H, W, pad)
+CASES = [
+    (3, 33, 31, 7, 7, 1), (17, 32, 64, 7, 7, 1), (1, 1, 1, 3, 3, 0), (2, 65, 40, 9, 11, 2),
+    (2, 24, 40, 28, 28, 1), (5, 40, 33, 14, 14, 1), (1, 64, 64, 56, 56, 1), (2, 8, 48, 12, 12, 0),
+    (2, 16, 16, 10, 14, 2), (1, 16, 32, 6, 150, 1), (1, 5, 7, 4, 261, 0), (1, 9, 6, 5, 140, 2),
+    (2, 3, 70, 33, 64, 1), (1, 640, 320, 16, 16, 1), (1, 320, 640, 16, 18, 1),
+    (2, 1280, 640, 8, 8, 1), (40, 4, 4, 5, 5, 2), (9, 96, 96, 1, 8, 1), (4, 30, 30, 8, 1, 1),
+]
+
+
+def weight_grad(x, dy, pad, C, K):
+    from nova_winograd.ops import check, get_lib
+
+    lib = get_lib()
+    B, _, H, W = x.shape
+    gw = torch.full((K, C, 3, 3), float("nan"), device=DEV)
+    h = lib.nova_create()
+    try:
+        lib.nova_set_stream(h, torch.cuda.current_stream().cuda_stream)
+        lib.nova_weight_grad(h, x.data_ptr(), dy.data_ptr(), gw.data_ptr(), B, C, K, H, W, pad, 0)
+        check()
+        torch.cuda.synchronize()
+    finally:
+        lib.nova_destroy(h)
+    return gw
+
+
+def exact(x, dy, pad):
+    """The gradient and sum |dY||x| per entry in fp64, tap by tap."""
+    K, C = dy.shape[1], x.shape[1]
+    Ho, Wo = dy.shape[2:]
+    xp = torch.nn.functional.pad(x.double(), (pad, pad, pad, pad)).transpose(0, 1)
+    g = dy.double().transpose(0, 1).reshape(K, -1)
+    want = torch.empty(K, C, 3, 3, dtype=torch.float64, device=x.device)
+    mag = torch.empty_like(want)
+    for r in range(3):
+        for s in range(3):
+            xs = xp[:, :, r:r + Ho, s:s + Wo].reshape(C, -1).t().contiguous()
+            want[:, :, r, s] = g @ xs
+            mag[:, :, r, s] = g.abs() @ xs.abs()
+    return want, mag
+
+
+def offset_copy(t, halves):
+    """t's values at an address `halves` fp16 elements past an allocation, with
+    NaN on both sides."""
+    buf = torch.full((t.numel() + halves + 8,), float("nan"), dtype=t.dtype, device=t.device)
+    buf[halves:halves + t.numel()] = t.reshape(-1)
+    return buf[halves:halves + t.numel()].view(t.shape)
+
+
+@pytest.mark.parametrize("B,C,K,H,W,pad", CASES)
+def test_direct_weight_grad(B, C, K, H, W, pad):
+    print(f"[wgrad direct] B={B} C={C} K={K} H={H} W={W} pad={pad}", flush=True)
+    g = torch.Generator().manual_seed(H * W + C)
+    x = torch.randn(B, C, H, W, generator=g).half().to(DEV)
+    # gradients down into fp16's subnormals
+    dy = (torch.randn(B, K, H + 2 * pad - 2, W + 2 * pad - 2, generator=g) * 1e-4).half().to(DEV)
+    want, mag = exact(x, dy, pad)
+    n = dy.numel() // K
+    got = weight_grad(x, dy, pad, C, K)
+    assert ((got.double() - want).abs() <= n * 2.0**-23 * mag + 1e-30).all()
+    # any address and any neighbours in memory: the same bits
+    for xo, go in ((1, 0), (0, 1), (3, 2)):
+        again = weight_grad(offset_copy(x, xo), offset_copy(dy, go), pad, C, K)
+        assert torch.equal(got, again)
+
+
+@pytest.mark.parametrize("W", [7, 12, 16])
+def test_infinities_stay_in_their_channels(W):
+    """An infinite x makes only its own input channel's taps infinite or NaN,
+    an infinite dY only its own output channel's: the chunks that reach past a
+    row or a channel hold zeros, not a neighbour's values."""
+    B, C, K, H = 2, 40, 40, 10
+    g = torch.Generator().manual_seed(W)
+    x = torch.randn(B, C, H, W, generator=g).half().to(DEV)
+    dy = torch.randn(B, K, H, W, generator=g).half().to(DEV)
+    base = weight_grad(x, dy, 1, C, K)
+    x2, dy2 = x.clone(), dy.clone()
+    x2[0, 5, 0, 0] = float("inf")
+    x2[1, 9, H - 1, W - 1] = float("-inf")
+    got = weight_grad(x2, dy, 1, C, K)
+    keep = torch.ones(C, dtype=torch.bool, device=DEV)
+    keep[[5, 9]] = False
+    assert torch.equal(got[:, keep], base[:, keep])
+    assert not torch.isfinite(got[:, 5, 0, 0]).any() and not torch.isfinite(got[:, 9, 2, 2]).any()
+    dy2[0, 3, H - 1, W - 1] = float("-inf")
+    got = weight_grad(x, dy2, 1, C, K)
+    keep = torch.arange(K, device=DEV) != 3
+    assert torch.equal(got[keep], base[keep])
+    assert not torch.isfinite(got[3, :, 0, 0]).any()
