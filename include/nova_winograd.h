@@ -115,6 +115,15 @@ NOVA_API const char* nova_get_last_error_message(void);
  * for bit. */
 NOVA_API void nova_set_weights_f16(nova_handle_t h, const void* d_weight_f16, int K, int C);
 
+/* No counterpart in the reference: the filter of a layer's input gradient.
+ * d_weight is the layer's w[C][K][3][3] (fp32, or fp16 when w_f16 = 1), read
+ * with both spatial axes reversed: the handle then holds what nova_set_weights
+ * (or nova_set_weights_f16) gives for w.flip(2, 3).transpose(0, 1), bit for
+ * bit, and its forward at padding 2 - p is the gradient. K and C are the
+ * handle's own: K = the layer's input channels. */
+NOVA_API void nova_set_weights_flipped(nova_handle_t h, const void* d_weight, int K, int C,
+                                       int w_f16);
+
 /* No counterpart in the reference's C-ABI: the weight gradient, which the
  * reference computes in fp32 PyTorch with a per-sample unfold loop
  * (/root/reference/nova_winograd/conv2d.py:121-147). d_grad_weight receives
@@ -128,6 +137,12 @@ NOVA_API void nova_set_weights_f16(nova_handle_t h, const void* d_weight_f16, in
 NOVA_API void nova_weight_grad(nova_handle_t h, const void* d_input, const void* d_grad_output,
                                void* d_grad_weight, int batch, int C, int K, int H, int W,
                                int pad, int grad_f32);
+/* nova_weight_grad and, into d_grad_bias (fp32, K values), the sums of
+ * d_grad_output over images and pixels, added in fp32. */
+NOVA_API void nova_weight_bias_grad(nova_handle_t h, const void* d_input,
+                                    const void* d_grad_output, void* d_grad_weight,
+                                    void* d_grad_bias, int batch, int C, int K, int H, int W,
+                                    int pad, int grad_f32);
 
 /* Stream for the handle's subsequent work (a hipStream_t; NULL = null stream). */
 NOVA_API void nova_set_stream(nova_handle_t h, void* stream);

@@ -180,6 +180,27 @@ bool ensure_ws(Handle* H, size_t bytes) {
     return true;
 }
 
+// Device memory for a fragment-ordered copy of U (32-bit offsets in the
+// kernels that read it).
+bool alloc_copy(Handle* H, uint16_t** copy, size_t* cap, const char* what) {
+    const size_t need = (size_t)u_frag_elems(H->K, H->Cp) * sizeof(uint16_t);
+    if ((int64_t)need >= ((int64_t)1 << 31)) {
+        set_error(kErrInvalidArgument, "%s of %lld bytes exceeds 2^31 - 1", what, (long long)need);
+        return false;
+    }
+    if (need <= *cap) return true;
+    if (*copy) {
+        if (!hip_ok(hipFree(*copy), "hipFree(filter copy)")) return false;
+        *copy = nullptr;
+        *cap = 0;
+    }
+    if (!hip_ok(hipMalloc(copy, need), "hipMalloc(filter copy)")) return false;
+    *cap = need;
+    return true;
+}
+bool alloc_uf(Handle* H) { return alloc_copy(H, &H->Uf, &H->Uf_cap, "fused filter copy"); }
+bool alloc_uw(Handle* H) { return alloc_copy(H, &H->Uw, &H->Uw_cap, "filter block copy"); }
+
 // The fragment-ordered copy of U that the fused kernels read, built from U
 // on the handle's stream the first time a fused path needs it for the
 // current weights (set_weights builds it at once when the automatic choice
@@ -188,21 +209,7 @@ bool ensure_ws(Handle* H, size_t bytes) {
 // hold it: for 1280 x 1280 channels that saves 210 MB per handle.
 bool ensure_uf(Handle* H) {
     if (H->uf_ready) return true;
-    const size_t need = (size_t)u_frag_elems(H->K, H->Cp) * sizeof(uint16_t);
-    if ((int64_t)need >= ((int64_t)1 << 31)) {  // 32-bit offsets in the fused kernels
-        set_error(kErrInvalidArgument, "fused filter copy of %lld bytes exceeds 2^31 - 1",
-                  (long long)need);
-        return false;
-    }
-    if (need > H->Uf_cap) {
-        if (H->Uf) {
-            if (!hip_ok(hipFree(H->Uf), "hipFree(Uf)")) return false;
-            H->Uf = nullptr;
-            H->Uf_cap = 0;
-        }
-        if (!hip_ok(hipMalloc(&H->Uf, need), "hipMalloc(Uf)")) return false;
-        H->Uf_cap = need;
-    }
+    if (!alloc_uf(H)) return false;
     H->uf_ready = hip_ok(launch_u_frag(H->U, H->Uf, H->K, H->Cp, H->stream),
                          "filter fragment order");
     return H->uf_ready;
@@ -214,21 +221,7 @@ bool ensure_uf(Handle* H) {
 // forced, else on the first forward that needs it.
 bool ensure_uw(Handle* H) {
     if (H->uw_ready) return true;
-    const size_t need = (size_t)u_frag_elems(H->K, H->Cp) * sizeof(uint16_t);
-    if ((int64_t)need >= ((int64_t)1 << 31)) {  // 32-bit offsets in the two-pass kernel
-        set_error(kErrInvalidArgument, "filter block copy of %lld bytes exceeds 2^31 - 1",
-                  (long long)need);
-        return false;
-    }
-    if (need > H->Uw_cap) {
-        if (H->Uw) {
-            if (!hip_ok(hipFree(H->Uw), "hipFree(Uw)")) return false;
-            H->Uw = nullptr;
-            H->Uw_cap = 0;
-        }
-        if (!hip_ok(hipMalloc(&H->Uw, need), "hipMalloc(Uw)")) return false;
-        H->Uw_cap = need;
-    }
+    if (!alloc_uw(H)) return false;
     H->uw_ready = hip_ok(launch_u_wfrag(H->U, H->Uw, H->K, H->Cp, H->stream),
                          "filter two-pass order");
     return H->uw_ready;
@@ -949,7 +942,7 @@ void nova_destroy(nova_handle_t h) {
 
 namespace {
 
-void set_weights_impl(nova_handle_t h, const void* d_weight, int K, int C, bool w_f16,
+void set_weights_impl(nova_handle_t h, const void* d_weight, int K, int C, bool w_f16, bool flip,
                       const char* fn) {
     Handle* H = as_handle(h, fn);
     if (!H) return;
@@ -983,6 +976,9 @@ void set_weights_impl(nova_handle_t h, const void* d_weight, int K, int C, bool 
         }
         H->U_cap = need;
     }
+    // new weights of the layer whose last ones got their operand blocks in a
+    // forward (or here) will need them again
+    const bool again = H->uw_ready && H->K == K && H->C == C;
     H->uf_ready = false;
     H->uw_ready = false;
     H->K = K;
@@ -996,13 +992,17 @@ void set_weights_impl(nova_handle_t h, const void* d_weight, int K, int C, bool 
             cus > 0)
             H->cus = cus;
     }
-    H->ready = hip_ok(launch_filter_transform_gemm(d_weight, w_f16, H->U, K, C, Cp, H->stream),
+    const bool uf = (C <= 64 && K <= 64 && H->path_pref == 0) || H->path_pref == 2 ||
+                    H->path_pref == 3 || H->path_pref == 5;
+    const bool uw =
+        again || H->path_pref == 6 || (H->path_pref == 0 && two_pass_possible(C, K));
+    H->ready = false;
+    if ((uf && !alloc_uf(H)) || (uw && !alloc_uw(H))) return;
+    H->ready = hip_ok(launch_filter_prep(d_weight, w_f16, flip, H->U, uf ? H->Uf : nullptr,
+                                         uw ? H->Uw : nullptr, K, C, Cp, H->cus, H->stream),
                       "filter transform");
-    const bool fused_possible = (C <= 64 && K <= 64 && H->path_pref == 0) ||
-                                H->path_pref == 2 || H->path_pref == 3 || H->path_pref == 5;
-    if (H->ready && fused_possible) H->ready = ensure_uf(H);
-    if (H->ready && (H->path_pref == 6 || (H->path_pref == 0 && two_pass_possible(C, K))))
-        H->ready = ensure_uw(H);
+    H->uf_ready = uf && H->ready;
+    H->uw_ready = uw && H->ready;
 }
 
 }  // namespace
@@ -1010,11 +1010,19 @@ void set_weights_impl(nova_handle_t h, const void* d_weight, int K, int C, bool 
 extern "C" {
 
 void nova_set_weights(nova_handle_t h, const void* d_weight, int K, int C) {
-    set_weights_impl(h, d_weight, K, C, false, "nova_set_weights");
+    set_weights_impl(h, d_weight, K, C, false, false, "nova_set_weights");
 }
 
 void nova_set_weights_f16(nova_handle_t h, const void* d_weight_f16, int K, int C) {
-    set_weights_impl(h, d_weight_f16, K, C, true, "nova_set_weights_f16");
+    set_weights_impl(h, d_weight_f16, K, C, true, false, "nova_set_weights_f16");
+}
+
+void nova_set_weights_flipped(nova_handle_t h, const void* d_weight, int K, int C, int w_f16) {
+    if (w_f16 != 0 && w_f16 != 1) {
+        set_error(kErrInvalidArgument, "nova_set_weights_flipped: w_f16 must be 0 or 1");
+        return;
+    }
+    set_weights_impl(h, d_weight, K, C, w_f16 != 0, true, "nova_set_weights_flipped");
 }
 
 void nova_forward(nova_handle_t h, const void* d_input, void* d_output, int batch, int H,
@@ -1059,15 +1067,19 @@ void nova_forward_workspace(nova_handle_t h, const void* d_input, void* d_output
                  64 * (int64_t)Hd->K * bp_user, "nova_forward_workspace");
 }
 
-void nova_weight_grad(nova_handle_t h, const void* d_input, const void* d_grad_output,
-                      void* d_grad_weight, int batch, int C, int K, int H, int W, int pad,
-                      int grad_f32) {
-    Handle* Hd = as_handle(h, "nova_weight_grad");
+}  // extern "C"
+
+namespace {
+
+void weight_grad_impl(nova_handle_t h, const void* d_input, const void* d_grad_output,
+                      void* d_grad_weight, void* d_grad_bias, int batch, int C, int K, int H,
+                      int W, int pad, int grad_f32, const char* fn) {
+    Handle* Hd = as_handle(h, fn);
     if (!Hd) return;
     if (d_grad_weight == nullptr || batch < 0 || C < 1 || K < 1 || H < 1 || W < 1 || pad < 0 ||
         (grad_f32 != 0 && grad_f32 != 1) || H + 2 * pad - 2 < 1 || W + 2 * pad - 2 < 1 ||
         (batch > 0 && (d_input == nullptr || d_grad_output == nullptr))) {
-        set_error(kErrInvalidArgument, "nova_weight_grad: bad arguments");
+        set_error(kErrInvalidArgument, "%s: bad arguments", fn);
         return;
     }
     int dev = 0, cus = 0;
@@ -1075,22 +1087,30 @@ void nova_weight_grad(nova_handle_t h, const void* d_input, const void* d_grad_o
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
         cus < 1)
         cus = 256;
-    if (!grad_f32) {
-        const WgradDirectPlan dp = wgrad_direct_plan(batch, C, K, H, W, pad, cus);
-        if (dp.ok) {
-            if (dp.ws_bytes > 0 && !ensure_ws(Hd, (size_t)dp.ws_bytes)) return;
-            hip_ok(launch_wgrad_direct(static_cast<const uint16_t*>(d_input),
-                                       static_cast<const uint16_t*>(d_grad_output),
-                                       static_cast<float*>(d_grad_weight), batch, C, K, H, W, pad,
-                                       dp, Hd->ws, Hd->stream),
-                   "weight gradient");
-            return;
-        }
+    WgradDirectPlan dp{};
+    if (!grad_f32) dp = wgrad_direct_plan(batch, C, K, H, W, pad, cus);
+    // the sums of dY per output channel: with the direct products, else a
+    // launch of their own
+    if (d_grad_bias != nullptr && !(dp.ok && dp.bias) &&
+        !hip_ok(launch_bias_grad(d_grad_output, grad_f32 != 0, static_cast<float*>(d_grad_bias),
+                                 batch, K, (int64_t)(H + 2 * pad - 2) * (W + 2 * pad - 2),
+                                 Hd->stream),
+                "bias gradient"))
+        return;
+    if (dp.ok) {
+        if (dp.ws_bytes > 0 && !ensure_ws(Hd, (size_t)dp.ws_bytes)) return;
+        hip_ok(launch_wgrad_direct(static_cast<const uint16_t*>(d_input),
+                                   static_cast<const uint16_t*>(d_grad_output),
+                                   static_cast<float*>(d_grad_weight),
+                                   dp.bias ? static_cast<float*>(d_grad_bias) : nullptr, batch, C,
+                                   K, H, W, pad, dp, Hd->ws, Hd->stream),
+               "weight gradient");
+        return;
     }
     const WgradPlan pl = wgrad_plan(batch, C, K, H, W, pad, cus);
     if (!pl.ok) {
         set_error(kErrInvalidArgument,
-                  "nova_weight_grad: one image of this shape exceeds the kernels' 32-bit offsets");
+                  "%s: one image of this shape exceeds the kernels' 32-bit offsets", fn);
         return;
     }
     if (!ensure_ws(Hd, (size_t)pl.ws_bytes)) return;
@@ -1098,6 +1118,28 @@ void nova_weight_grad(nova_handle_t h, const void* d_input, const void* d_grad_o
                         static_cast<float*>(d_grad_weight), batch, C, K, H, W, pad, pl, Hd->ws,
                         Hd->stream),
            "weight gradient");
+}
+
+}  // namespace
+
+extern "C" {
+
+void nova_weight_grad(nova_handle_t h, const void* d_input, const void* d_grad_output,
+                      void* d_grad_weight, int batch, int C, int K, int H, int W, int pad,
+                      int grad_f32) {
+    weight_grad_impl(h, d_input, d_grad_output, d_grad_weight, nullptr, batch, C, K, H, W, pad,
+                     grad_f32, "nova_weight_grad");
+}
+
+void nova_weight_bias_grad(nova_handle_t h, const void* d_input, const void* d_grad_output,
+                           void* d_grad_weight, void* d_grad_bias, int batch, int C, int K, int H,
+                           int W, int pad, int grad_f32) {
+    if (d_grad_bias == nullptr) {
+        set_error(kErrInvalidArgument, "nova_weight_bias_grad: null bias gradient");
+        return;
+    }
+    weight_grad_impl(h, d_input, d_grad_output, d_grad_weight, d_grad_bias, batch, C, K, H, W, pad,
+                     grad_f32, "nova_weight_bias_grad");
 }
 
 void nova_compute_tiling(int H, int W, int pad, int* nh, int* nw, int* H_out, int* W_out) {

@@ -99,9 +99,12 @@ inline int64_t dword_ceil(int64_t bytes) { return (bytes + 3) & ~(int64_t)3; }
 // Reference layout: U[p][c][k] (U[p*K*C + c*K + k]).
 hipError_t launch_filter_transform_ref(const float* w, uint16_t* U, int K, int C,
                                        hipStream_t s);
-// Product layout: U[p][k][Cp], zero for c >= C (Cp = pad8(C)).
-hipError_t launch_filter_transform_gemm(const void* w, bool w_f16, uint16_t* U, int K, int C,
-                                        int Cp, hipStream_t s);
+// Product layout U[p][k][Cp], zero for c >= C (Cp = pad8(C)), and the
+// fragment-ordered copies Uf and Uw below where they are not null. flip: w is
+// [C][K][3][3], read with both spatial axes reversed (the filter of the input
+// gradient of the layer with weights w).
+hipError_t launch_filter_prep(const void* w, bool w_f16, bool flip, uint16_t* U, uint16_t* Uf,
+                              uint16_t* Uw, int K, int C, int Cp, int cus, hipStream_t s);
 
 // Fragment-ordered copy of U for the fused kernels: for each position p,
 // 16-row output-channel tile kt and 32-channel chunk j, one
@@ -310,12 +313,17 @@ struct WgradDirectPlan {
     int Ws, nstrip;     // 8-pixel segments per column strip, strips per row
     int lo, XS, XP, xpitch, dpitch, dstart, zero, nblk, nwx;  // LDS geometry (16-byte chunks)
     int ntk, nt, nunits, nsplit;
-    int64_t ws_bytes;   // the splits' partial filters (none with one split)
+    int64_t ws_bytes;   // the splits' partial filters and sums (none with one split)
+    bool bias;          // the kernel can also sum dY per output channel
     bool ok;
 };
 WgradDirectPlan wgrad_direct_plan(int B, int C, int K, int H, int W, int pad, int cus);
-hipError_t launch_wgrad_direct(const uint16_t* x, const uint16_t* dy, float* dw, int B, int C,
-                               int K, int H, int W, int pad, const WgradDirectPlan& plan,
+// db: fp32 sums of dY per output channel, or null (plan.bias: pads 0 and 1).
+hipError_t launch_wgrad_direct(const uint16_t* x, const uint16_t* dy, float* dw, float* db, int B,
+                               int C, int K, int H, int W, int pad, const WgradDirectPlan& plan,
                                void* ws, hipStream_t s);
+// db[k] = sum of dY over images and pixels (fp16, or fp32 if dy_f32), fp32.
+hipError_t launch_bias_grad(const void* dy, bool dy_f32, float* db, int B, int K, int64_t HoWo,
+                            hipStream_t s);
 
 }  // namespace nova

@@ -75,17 +75,147 @@ hipError_t launch_filter_transform_ref(const float* w, uint16_t* U, int K, int C
     return hipGetLastError();
 }
 
-hipError_t launch_filter_transform_gemm(const void* w, bool w_f16, uint16_t* U, int K, int C,
-                                        int Cp, hipStream_t s) {
-    const int64_t n = (int64_t)K * Cp;
-    const int64_t blocks = (n + 255) / 256;
-    if (w_f16)
-        launch(filter_transform_kernel<false, _Float16>, dim3((unsigned)blocks), dim3(256), s,
-            static_cast<const _Float16*>(w), reinterpret_cast<_Float16*>(U), K, C, Cp);
+// Filter transform into everything a layer's kernels read, in one launch: the
+// product layout U[p][k][Cp] and, where not null, the two fragment-ordered
+// copies (launch_u_frag's Uf, launch_u_wfrag's Uw) with their zero padding.
+// kFlip: the filter of the input gradient, read from the layer's own weights
+// [C][K][3][3] with both spatial axes reversed.
+//
+// Workgroup: 8 waves, wave r computes row r of the 8 x 8 positions; a lane
+// holds CPT consecutive channels of one k, 64 lanes 16 such groups (or all of
+// a small layer's) by some k; the 8 waves share the tile's weights in LDS
+// (read by each lane for itself, 288 bytes apart, they cost 38 us at 512 x 512
+// against 12). CPT 8 (16-byte stores) where that fills the chip, else 2. Bound
+// at small layers by one load, one barrier and one store round trip, at large
+// ones by the 90 VALU operations a position row takes per channel (the chain's
+// nine terms, unfolded: the order of the rounding is the contract). Measured
+// on MI355X (us, kernels before -> this one): 64 x 64 with both copies 3.8 +
+// 2.5 + 2.5 -> 4.2, 128 x 128 with Uw 4.1 + 2.8 -> 4.2; flipped, where torch
+// first reversed and transposed the weights, 512 x 512 6.9 + 10.8 + 11.1 ->
+// 11.7, 320 x 320 5.2 + 6.4 + 6.0 -> 8.2. U alone, unflipped, stays with
+// filter_transform_kernel, whose many small workgroups overlap better (256 x
+// 256 4.8 against 5.7, 1280 x 1280 47 against 71).
+template <typename WT, int CPT, bool kFlip>
+__global__ __launch_bounds__(512) void filter_prep_kernel(
+    const WT* __restrict__ w, _Float16* __restrict__ U, _Float16* __restrict__ Uf,
+    _Float16* __restrict__ Uw, int K, int C, int Cp, int kdom, int groups, int cshift, int ncb,
+    int nkt, int nkp) {
+    constexpr int kLane = 9 * CPT + 1;  // floats of a lane's filters in LDS, odd: no conflicts
+    __shared__ float ws[64 * kLane];
+    const int lane = threadIdx.x & 63;
+    const int r = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int cb = (int)blockIdx.x % ncb, kb = (int)blockIdx.x / ncb;
+    const int cg0 = cb << cshift, kk0 = kb << (6 - cshift);
+    // the tile's filters, read along memory: a row of taps of one k over the
+    // tile's channels (of one channel over the tile's k when flipped)
+    const int cw = CPT << cshift, kw = 64 >> cshift;
+    for (int n = threadIdx.x; n < 64 * CPT * 9; n += 512) {
+        const int run = kFlip ? 9 * kw : 9 * cw;
+        const int row = n / 9 >> (kFlip ? 6 - cshift : cshift + (CPT == 8 ? 3 : 1));
+        const int i = (n - row * run) / 9, tap = n - row * run - 9 * i;
+        const int kl = kFlip ? i : row, cl = kFlip ? row : i;
+        const int k = kk0 + kl, c = cg0 * CPT + cl;
+        // fp16 weights widen to fp32 exactly: the same U as their fp32 copy
+        float v = 0.0f;
+        if (k < K && c < C)
+            v = (float)w[(kFlip ? (int64_t)c * K + k : (int64_t)k * C + c) * 9 + tap];
+        ws[((kl << cshift) + cl / CPT) * kLane + (cl % CPT) * 9 + (kFlip ? 8 - tap : tap)] = v;
+    }
+    __syncthreads();
+    const int cg = cg0 + (lane & ((1 << cshift) - 1));
+    const int k = kk0 + (lane >> cshift);
+    if (k >= kdom || cg >= groups) return;
+    const int c0 = cg * CPT;
+    const float g[3] = {kG[r][0], kG[r][1], kG[r][2]};
+    float u[CPT][8];
+#pragma unroll
+    for (int e = 0; e < CPT; e++) {
+        float t[3][3];
+#pragma unroll
+        for (int i = 0; i < 9; i++) t[i / 3][i % 3] = g[i / 3] * ws[lane * kLane + e * 9 + i];
+#pragma unroll
+        for (int s = 0; s < 8; s++) {  // filter_tile's chain
+            float acc = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 9; i++) acc = __builtin_fmaf(t[i / 3][i % 3], kG[s][i % 3], acc);
+            u[e][s] = acc;
+        }
+    }
+    typedef unsigned uv __attribute__((ext_vector_type(CPT / 2)));
+    const int kt = k >> 4, j = c0 >> 5;
+#pragma unroll
+    for (int s = 0; s < 8; s++) {
+        uv v;
+#pragma unroll
+        for (int e = 0; e < CPT / 2; e++) v[e] = pack_f16x2(u[2 * e][s], u[2 * e + 1][s]);
+        const int64_t p = 8 * r + s;
+        if (k < K && c0 < Cp) *reinterpret_cast<uv*>(U + (p * K + k) * Cp + c0) = v;
+        const int64_t blk = ((p * nkt + kt) * nkp + j) * 512;
+        if (Uw != nullptr)
+            *reinterpret_cast<uv*>(Uw + blk + ((k & 15) + 16 * ((c0 & 31) >> 3)) * 8 + (c0 & 7)) =
+                v;
+        if (Uf != nullptr) {
+            // 4-channel slots: lane (k % 16) + 16 * (c % 16 / 4), half c % 32 / 16
+            auto slot = [&](int c) {
+                return Uf + blk + ((k & 15) + 16 * ((c & 15) >> 2)) * 8 + ((c & 31) >> 4) * 4 +
+                       (c & 3);
+            };
+            if constexpr (CPT == 8) {
+                typedef unsigned u2 __attribute__((ext_vector_type(2)));
+                *reinterpret_cast<u2*>(slot(c0)) = u2{v[0], v[1]};
+                *reinterpret_cast<u2*>(slot(c0 + 4)) = u2{v[2], v[3]};
+            } else {
+                *reinterpret_cast<uv*>(slot(c0)) = v;
+            }
+        }
+    }
+}
+
+template <typename WT, int CPT>
+static hipError_t launch_prep(const WT* w, bool flip, uint16_t* U, uint16_t* Uf, uint16_t* Uw,
+                              int K, int C, int Cp, hipStream_t s) {
+    const int nkt = (K + 15) / 16, nkp = (Cp + 31) / 32;
+    const bool frags = Uf != nullptr || Uw != nullptr;  // padded to 16 rows and 32 channels
+    const int kdom = frags ? 16 * nkt : K, groups = (frags ? 32 * nkp : Cp) / CPT;
+    int cshift = 0;  // channel groups per tile: 16, or a small layer's all
+    while (cshift < 4 && (1 << cshift) < groups) cshift++;
+    const int ncb = (groups + (1 << cshift) - 1) >> cshift;
+    const int kpt = 64 >> cshift;
+    const dim3 grid((unsigned)(ncb * ((kdom + kpt - 1) / kpt)));
+    auto* const u = reinterpret_cast<_Float16*>(U);
+    auto* const uf = reinterpret_cast<_Float16*>(Uf);
+    auto* const uw = reinterpret_cast<_Float16*>(Uw);
+    if (flip)
+        launch(filter_prep_kernel<WT, CPT, true>, grid, dim3(512), s, w, u, uf, uw, K, C, Cp, kdom,
+               groups, cshift, ncb, nkt, nkp);
     else
-        launch(filter_transform_kernel<false, float>, dim3((unsigned)blocks), dim3(256), s,
-            static_cast<const float*>(w), reinterpret_cast<_Float16*>(U), K, C, Cp);
+        launch(filter_prep_kernel<WT, CPT, false>, grid, dim3(512), s, w, u, uf, uw, K, C, Cp,
+               kdom, groups, cshift, ncb, nkt, nkp);
     return hipGetLastError();
+}
+
+hipError_t launch_filter_prep(const void* w, bool w_f16, bool flip, uint16_t* U, uint16_t* Uf,
+                              uint16_t* Uw, int K, int C, int Cp, int cus, hipStream_t s) {
+    if (!flip && Uf == nullptr && Uw == nullptr) {
+        const dim3 grid((unsigned)(((int64_t)K * Cp + 255) / 256));
+        if (w_f16)
+            launch(filter_transform_kernel<false, _Float16>, grid, dim3(256), s,
+                   static_cast<const _Float16*>(w), reinterpret_cast<_Float16*>(U), K, C, Cp);
+        else
+            launch(filter_transform_kernel<false, float>, grid, dim3(256), s,
+                   static_cast<const float*>(w), reinterpret_cast<_Float16*>(U), K, C, Cp);
+        return hipGetLastError();
+    }
+    // 16-byte stores where their tiles (64 lanes x 8 channels) fill the chip
+    const bool wide = (int64_t)K * Cp >= (int64_t)512 * cus;
+    if (w_f16) {
+        const auto* h = static_cast<const _Float16*>(w);
+        return wide ? launch_prep<_Float16, 8>(h, flip, U, Uf, Uw, K, C, Cp, s)
+                    : launch_prep<_Float16, 2>(h, flip, U, Uf, Uw, K, C, Cp, s);
+    }
+    const auto* f = static_cast<const float*>(w);
+    return wide ? launch_prep<float, 8>(f, flip, U, Uf, Uw, K, C, Cp, s)
+                : launch_prep<float, 2>(f, flip, U, Uf, Uw, K, C, Cp, s);
 }
 
 // Reorder U[p][k][Cp] into the fused kernels' A-operand order (zero padded),

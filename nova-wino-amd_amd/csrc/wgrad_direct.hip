@@ -67,7 +67,8 @@ enum Stage { kRegs, kDirect, kDirectTail };
 struct WdArgs {
     const char* x;
     const char* dy;
-    float* out;
+    float* out;             // dw, or the splits' partial filters
+    float* bias;            // sums of dY: db, or the splits' partial sums; null: none
     int64_t x_bytes, dy_bytes;
     int B, C, K, H, W, Ho, Wo;
     int G, R, nrb;          // images and x rows per unit, row blocks per image
@@ -255,6 +256,11 @@ __global__ __launch_bounds__(kThreads) void wgrad_direct_kernel(WdArgs a) {
 #pragma unroll
         for (int e = 0; e < 16; e++) acc[t][e] = 0.0f;
 
+    // sums of dY: waves of the first input-channel tile, each lane its row's
+    // pixels of the steps it multiplies (tap r = 1 meets every dY row once)
+    const bool sums = PAD < 2 && a.bias != nullptr && c0 == 0 && wc == 0;
+    float bsum[2] = {0.0f, 0.0f}, bunit = 0.0f;  // a unit's, all units'
+
     const int l32 = lane & 31, g = lane >> 5;
     const int xrow = (wc * 32 + l32) * a.xpitch + 1 + a.lo;
     const int drow = a.dstart + (wk * 32 + l32) * a.dpitch;
@@ -294,6 +300,10 @@ __global__ __launch_bounds__(kThreads) void wgrad_direct_kernel(WdArgs a) {
             }
         };
         auto multiply = [&](const Frag& f) {
+            if (sums) {
+#pragma unroll
+                for (int i = 0; i < 8; i++) bsum[i & 1] += (float)__builtin_bit_cast(h8, f.d[1])[i];
+            }
 #pragma unroll
             for (int s = 0; s < 3; s++) {
                 // halves s - PAD .. s - PAD + 7 around the segment
@@ -333,6 +343,10 @@ __global__ __launch_bounds__(kThreads) void wgrad_direct_kernel(WdArgs a) {
                 __builtin_amdgcn_sched_barrier(0);
                 multiply(f1);
             }
+        }
+        if (sums) {
+            bunit += bsum[0] + bsum[1];
+            bsum[0] = bsum[1] = 0.0f;
         }
         advance(up);
     };
@@ -406,6 +420,21 @@ __global__ __launch_bounds__(kThreads) void wgrad_direct_kernel(WdArgs a) {
     float* const red[3] = {reinterpret_cast<float*>(buf0), reinterpret_cast<float*>(buf1),
                            reinterpret_cast<float*>(buf2)};
     float* const out = a.out + (int64_t)sp * a.K * a.C * 9;
+    if (PAD < 2 && a.bias != nullptr && c0 == 0) {
+        if (wc == 0) red[0][wave * 64 + lane] = bunit;
+        barrier();
+        if (tid < 32 * WK && k0 + tid < a.K) {
+            const int w0 = tid >> 5;  // the wave with this row, wc = 0 and wp = 0
+            float v = 0.0f;
+            for (int p = 0; p < WP; p++) {
+                const float* r = red[0] + (w0 + p * WK * WC) * 64 + (tid & 31);
+                v += r[0];
+                v += r[32];
+            }
+            a.bias[(int64_t)sp * a.K + k0 + tid] = v;
+        }
+        barrier();
+    }
 #pragma unroll
     for (int q = 0; q < 4; q++) {
 #pragma unroll
@@ -431,31 +460,56 @@ __global__ __launch_bounds__(kThreads) void wgrad_direct_kernel(WdArgs a) {
     }
 }
 
-// dw[i] = sum over splits of part[s][i], in split order.
+// dw[i] = sum over splits of part[s][i], in split order, for n filter entries
+// and then nb bias entries (bpart[s][i] into db).
 constexpr int kRedThreads = 256;
 __global__ __launch_bounds__(kRedThreads) void wgrad_direct_reduce_kernel(
-    const float* __restrict__ part, float* __restrict__ dw, int64_t n, int nsplit) {
+    const float* __restrict__ part, float* __restrict__ dw, const float* __restrict__ bpart,
+    float* __restrict__ db, int64_t n, int nb, int nsplit) {
     const int64_t i = (int64_t)blockIdx.x * kRedThreads + threadIdx.x;
-    if (i >= n) return;
-    const float* p = part + i;
+    if (i >= n + nb) return;
+    const bool filter = i < n;
+    const float* p = filter ? part + i : bpart + (i - n);
+    const int64_t ld = filter ? n : nb;
     float v = 0.0f;
     int s = 0;
     for (; s + 16 <= nsplit; s += 16) {
         float r[16];
 #pragma unroll
-        for (int u = 0; u < 16; u++) r[u] = p[(s + u) * n];
+        for (int u = 0; u < 16; u++) r[u] = p[(s + u) * ld];
 #pragma unroll
         for (int u = 0; u < 16; u++) v += r[u];
     }
     for (; s + 4 <= nsplit; s += 4) {
         float r[4];
 #pragma unroll
-        for (int u = 0; u < 4; u++) r[u] = p[(s + u) * n];
+        for (int u = 0; u < 4; u++) r[u] = p[(s + u) * ld];
 #pragma unroll
         for (int u = 0; u < 4; u++) v += r[u];
     }
-    for (; s < nsplit; s++) v += p[s * n];
-    dw[i] = v;
+    for (; s < nsplit; s++) v += p[s * ld];
+    (filter ? dw[i] : db[i - n]) = v;
+}
+
+// db[k] = sum of dY[b][k][:] over images and pixels, in fp64, rounded once:
+// one workgroup per channel.
+template <typename T>
+__global__ __launch_bounds__(256) void bias_grad_kernel(const T* __restrict__ dy,
+                                                        float* __restrict__ db, int B, int K,
+                                                        int64_t HoWo) {
+    __shared__ double s[256];
+    const int k = (int)blockIdx.x, tid = threadIdx.x;
+    double v = 0.0;
+    for (int b = 0; b < B; b++) {
+        const T* p = dy + ((int64_t)b * K + k) * HoWo;
+        for (int64_t i = tid; i < HoWo; i += 256) v += (double)p[i];
+    }
+    s[tid] = v;
+    for (int d = 128; d > 0; d >>= 1) {
+        __syncthreads();
+        if (tid < d) s[tid] += s[tid + d];
+    }
+    if (tid == 0) db[k] = (float)s[0];
 }
 
 inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
@@ -544,7 +598,7 @@ WgradDirectPlan wgrad_direct_plan(int B, int C, int K, int H, int W, int pad, in
                     // splits: one round of workgroups over the CUs
                     int64_t ns = std::max<int64_t>(1, cus / p.nt);
                     ns = std::min<int64_t>(ns, p.nunits);
-                    while (ns > 1 && 36 * ns * (int64_t)K * C >= ((int64_t)1 << 31)) ns--;
+                    while (ns > 1 && 4 * ns * K * (9 * (int64_t)C + 1) >= ((int64_t)1 << 31)) ns--;
                     p.nsplit = (int)ns;
                     const double rounds =
                         ceil_div((int)std::min<int64_t>(p.nt * ns, 1 << 30), cus);
@@ -564,7 +618,10 @@ WgradDirectPlan wgrad_direct_plan(int B, int C, int K, int H, int W, int pad, in
             if (Ws == wseg) break;
         }
     }
-    if (best.ok) best.ws_bytes = best.nsplit > 1 ? 36 * (int64_t)best.nsplit * K * C : 0;
+    // pad 2: no tap meets every dY row
+    best.bias = best.ok && pad < 2;
+    if (best.ok)
+        best.ws_bytes = best.nsplit > 1 ? 4 * (int64_t)best.nsplit * K * (9 * (int64_t)C + 1) : 0;
     return best;
 }
 
@@ -588,14 +645,28 @@ static hipError_t launch_pad(const WdArgs& a, const WgradDirectPlan& p, int stag
     return launch_direct<PAD, 2, 2>(a, stage, s);
 }
 
-hipError_t launch_wgrad_direct(const uint16_t* x, const uint16_t* dy, float* dw, int B, int C,
-                               int K, int H, int W, int pad, const WgradDirectPlan& p, void* ws,
-                               hipStream_t s) {
+hipError_t launch_bias_grad(const void* dy, bool dy_f32, float* db, int B, int K, int64_t HoWo,
+                            hipStream_t s) {
+    if (dy_f32)
+        launch(bias_grad_kernel<float>, dim3((unsigned)K), dim3(256), s,
+               static_cast<const float*>(dy), db, B, K, HoWo);
+    else
+        launch(bias_grad_kernel<_Float16>, dim3((unsigned)K), dim3(256), s,
+               static_cast<const _Float16*>(dy), db, B, K, HoWo);
+    return hipGetLastError();
+}
+
+hipError_t launch_wgrad_direct(const uint16_t* x, const uint16_t* dy, float* dw, float* db, int B,
+                               int C, int K, int H, int W, int pad, const WgradDirectPlan& p,
+                               void* ws, hipStream_t s) {
     const int Ho = H + 2 * pad - 2, Wo = W + 2 * pad - 2;
     WdArgs a{};
     a.x = reinterpret_cast<const char*>(x);
     a.dy = reinterpret_cast<const char*>(dy);
-    a.out = p.nsplit > 1 ? static_cast<float*>(ws) : dw;
+    float* const part = static_cast<float*>(ws);
+    float* const bpart = part + (int64_t)p.nsplit * 9 * K * C;
+    a.out = p.nsplit > 1 ? part : dw;
+    a.bias = db != nullptr && p.nsplit > 1 ? bpart : db;
     a.x_bytes = 2 * (int64_t)B * C * H * W;
     a.dy_bytes = 2 * (int64_t)B * K * Ho * Wo;
     a.B = B;
@@ -639,8 +710,11 @@ hipError_t launch_wgrad_direct(const uint16_t* x, const uint16_t* dy, float* dw,
                               : launch_pad<2>(a, p, stage, s);
     if (e != hipSuccess || p.nsplit == 1) return e;
     const int64_t n = (int64_t)9 * K * C;
-    launch(wgrad_direct_reduce_kernel, dim3((unsigned)((n + kRedThreads - 1) / kRedThreads)),
-           dim3(kRedThreads), s, static_cast<const float*>(ws), dw, n, p.nsplit);
+    const int nb = db != nullptr ? K : 0;
+    launch(wgrad_direct_reduce_kernel,
+           dim3((unsigned)((n + nb + kRedThreads - 1) / kRedThreads)), dim3(kRedThreads), s,
+           static_cast<const float*>(part), dw, static_cast<const float*>(bpart), db, n, nb,
+           p.nsplit);
     return hipGetLastError();
 }
 

@@ -5,7 +5,7 @@ Classes:
     NovaWinogradConv2d           inference module: cached filter transform,
                                  weight versioning, workspace caching
     NovaWinogradConv2dTrainable  HIP forward and backward (grad input through the
-                                 forward kernels, grad weight on the Winograd domain)
+                                 forward kernels, grad weight and bias in one pass)
     NovaWinogradConv2dCompilable ``torch.compile`` through the custom op
                                  ``torch.ops.nova.winograd_conv2d`` (bias fused)
 
@@ -179,6 +179,17 @@ class _Handle:
             self.lib.nova_set_weights(self.h, ptr(w), w.shape[0], w.shape[1])
         check("set_weights")
 
+    def set_weights_flipped(self, weight):
+        """The filter of the input gradient of a layer with ``weight``
+        [K, C, 3, 3]: what ``set_weights(weight.flip(2, 3).transpose(0, 1))``
+        gives, read from the layer's own weights in the one launch that
+        transforms them."""
+        w = weight.detach()
+        f16 = w.dtype == torch.float16
+        w = w.contiguous() if f16 else w.to(torch.float32).contiguous()
+        self.lib.nova_set_weights_flipped(self.h, ptr(w), w.shape[1], w.shape[0], int(f16))
+        check("set_weights")
+
     def __del__(self):
         try:
             if self.h and not _exiting:
@@ -268,7 +279,7 @@ def _grad_input_nova(holder, go, weight, padding, dtype):
     key = (weight.data_ptr(), weight._version, tuple(weight.shape), weight.dtype)
     ref = hd.key
     if not (ref is not None and ref[0]() is weight and ref[1] == key):
-        hd.set_weights(weight.detach().flip(2, 3).transpose(0, 1))
+        hd.set_weights_flipped(weight)
         hd.key = (weakref.ref(weight), key)
     g16 = go.to(torch.float16).contiguous()
     B, K, Ho, Wo = g16.shape
@@ -291,14 +302,14 @@ def _bwd_handle(holder):
     return hd
 
 
-def _grad_weight(holder, inp, go, weight, padding):
-    """dL/dw on the HIP path (nova_weight_grad): the Winograd-domain
-    products of the transformed input and the transformed output gradient,
-    reduced over the tiles and mapped back through G, all in fp32 -- in place
-    of the reference's per-sample fp32 unfold loop
-    (/root/reference/nova_winograd/conv2d.py:121-147). The input is the fp16
-    tensor the forward convolved, so this is the gradient of the forward as
-    computed."""
+def _grad_weight(holder, inp, go, weight, padding, bias=None):
+    """dL/dw on the HIP path (nova_weight_grad): for the float16 gradients that
+    autograd delivers, direct products of the input and the output gradient
+    over the pixels with fp32 sums -- in place of the reference's per-sample
+    fp32 unfold loop (/root/reference/nova_winograd/conv2d.py:121-147). The
+    input is the fp16 tensor the forward convolved, so this is the gradient of
+    the forward as computed. With ``bias``, returns (dL/dw, dL/dbias), the
+    latter summed by the same launches (nova_weight_bias_grad)."""
     hd = _bwd_handle(holder)
     hd.set_stream(go.device)
     x16 = inp.detach().to(torch.float16).contiguous()
@@ -309,10 +320,16 @@ def _grad_weight(holder, inp, go, weight, padding):
     B, C, H, W = x16.shape
     K = weight.shape[0]
     gw = torch.empty(K, C, 3, 3, dtype=torch.float32, device=go.device)
-    hd.lib.nova_weight_grad(hd.h, ptr(x16), ptr(g), ptr(gw), B, C, K, H, W, padding,
-                            1 if g.dtype == torch.float32 else 0)
-    check("backward (grad weight)")
-    return gw.to(weight.dtype)
+    f32 = 1 if g.dtype == torch.float32 else 0
+    if bias is None:
+        hd.lib.nova_weight_grad(hd.h, ptr(x16), ptr(g), ptr(gw), B, C, K, H, W, padding, f32)
+        check("backward (grad weight)")
+        return gw.to(weight.dtype)
+    gb = torch.empty(K, dtype=torch.float32, device=go.device)
+    hd.lib.nova_weight_bias_grad(hd.h, ptr(x16), ptr(g), ptr(gw), ptr(gb), B, C, K, H, W, padding,
+                                 f32)
+    check("backward (grad weight and bias)")
+    return gw.to(weight.dtype), gb.to(bias.dtype)
 
 
 class _BackwardHandles:
@@ -407,8 +424,7 @@ def _register_custom_op():
 
 class NovaWinogradFunction(torch.autograd.Function):
     """HIP forward; backward: grad input through the HIP forward (flipped
-    filter), grad weight through nova_weight_grad (fp32, Winograd domain),
-    grad bias a channel sum."""
+    filter), grad weight and grad bias through nova_weight_bias_grad."""
 
     @staticmethod
     def forward(ctx, input, weight, bias, padding, handle_holder):
@@ -426,9 +442,12 @@ class NovaWinogradFunction(torch.autograd.Function):
         go = grad_output.contiguous()
         if ctx.needs_input_grad[0]:
             grad_input = _grad_input_nova(ctx.holder, go, weight, padding, input.dtype)
-        if ctx.needs_input_grad[1]:
+        needs_bias = bias is not None and ctx.needs_input_grad[2]
+        if ctx.needs_input_grad[1] and needs_bias:
+            grad_weight, grad_bias = _grad_weight(ctx.holder, input, go, weight, padding, bias)
+        elif ctx.needs_input_grad[1]:
             grad_weight = _grad_weight(ctx.holder, input, go, weight, padding)
-        if bias is not None and ctx.needs_input_grad[2]:
+        elif needs_bias:
             grad_bias = go.float().sum(dim=(0, 2, 3)).to(bias.dtype)
         return grad_input, grad_weight, grad_bias, None, None
 

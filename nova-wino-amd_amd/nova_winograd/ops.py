@@ -56,12 +56,14 @@ _SIGNATURES = {
     "nova_set_window_bytes": (None, [_vp, ctypes.c_longlong]),
     "nova_set_epilogue": (None, [_vp, _vp, _i]),
     "nova_set_weights_f16": (None, [_vp, _vp, _i, _i]),
+    "nova_set_weights_flipped": (None, [_vp, _vp, _i, _i, _i]),
     "nova_set_residual": (None, [_vp, _vp]),
     "nova_set_layout": (None, [_vp, _i]),
     "nova_get_last_path": (_i, [_vp]),
     "nova_workspace_bytes": (ctypes.c_longlong, [_vp, _i, _i, _i, _i]),
     "nova_forward_noalloc": (None, [_vp, _vp, _vp, _i, _i, _i, _i]),
     "nova_weight_grad": (None, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i]),
+    "nova_weight_bias_grad": (None, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i]),
     "nova_profile_enable": (None, [_vp, _i]),
     "nova_profile_read": (_i, [_vp, ctypes.POINTER(ctypes.c_double),
                                ctypes.POINTER(ctypes.c_longlong)]),

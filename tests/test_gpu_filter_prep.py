@@ -1,0 +1,104 @@
+"""The one-launch filter preparation: U in the product layout against the
+oracle's transform, the flipped form against the flipped weights, and both
+fragment-ordered copies against U, at both lane widths (8 channels per lane
+from 512 pairs per CU on, else 2) and at channel counts off the 8, 16, 32 and
+64 blocks. The forwards of the paths that read each copy must agree bit for
+bit with the three-pass path, which reads U."""
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = torch.device("cuda:0")
+
+
+class DeviceView:
+    """The handle's U as an array torch can wrap without a copy."""
+
+    def __init__(self, ptr, shape):
+        self.__cuda_array_interface__ = {"shape": shape, "typestr": "<f2", "data": (ptr, False),
+                                         "version": 2}
+
+
+def handle_u(lib, h, K, C):
+    torch.cuda.synchronize()
+    return torch.as_tensor(DeviceView(lib.nova_get_U_gemm(h), (64, K, (C + 7) // 8 * 8)),
+                           device=DEV).clone()
+
+
+@pytest.mark.parametrize("K,C", [(1, 1), (3, 5), (16, 8), (17, 33), (64, 64), (72, 100),
+                                 (130, 24), (24, 130), (500, 264), (264, 500), (520, 256)])
+@pytest.mark.parametrize("f16", [False, True])
+def test_u_and_flipped_u(oracle, K, C, f16):
+    from nova_winograd.ops import check, get_lib
+
+    print(f"[filter prep] K={K} C={C} f16={f16}", flush=True)
+    lib = get_lib()
+    g = torch.Generator().manual_seed(K + C)
+    w = torch.randn(K, C, 3, 3, generator=g) * 0.1
+    w = w.half() if f16 else w
+    # off a 16-byte address, as a view into a larger parameter may be
+    buf = torch.zeros(w.numel() + 3, dtype=w.dtype, device=DEV)
+    buf[3:] = w.reshape(-1).to(DEV)
+    wd = buf[3:]
+    h, hf, hs = lib.nova_create(), lib.nova_create(), lib.nova_create()
+    try:
+        (lib.nova_set_weights_f16 if f16 else lib.nova_set_weights)(h, wd.data_ptr(), K, C)
+        check()
+        u = handle_u(lib, h, K, C)
+        want = oracle.filter_transform(w.float().numpy())  # [64][C][K]
+        want = torch.from_numpy(np.ascontiguousarray(want).view(np.float16)).to(DEV)
+        assert torch.equal(u[:, :, :C].view(torch.int16),
+                           want.reshape(64, C, K).transpose(1, 2).contiguous().view(torch.int16))
+        assert not u[:, :, C:].any()
+        lib.nova_set_weights_flipped(hf, wd.data_ptr(), C, K, 1 if f16 else 0)
+        check()
+        wf = w.flip(2, 3).transpose(0, 1).contiguous().to(DEV)
+        (lib.nova_set_weights_f16 if f16 else lib.nova_set_weights)(hs, wf.data_ptr(), C, K)
+        check()
+        assert torch.equal(handle_u(lib, hf, C, K).view(torch.int16),
+                           handle_u(lib, hs, C, K).view(torch.int16))
+    finally:
+        for x in (h, hf, hs):
+            lib.nova_destroy(x)
+
+
+@pytest.mark.parametrize("K,C", [(64, 64), (40, 48), (17, 9), (128, 128), (256, 128), (96, 24),
+                                 (512, 512)])
+def test_copies_match_u(K, C):
+    """Paths that read Uf (5, 3) or Uw (6, 7) against path 1, with weights set
+    twice: the second time a handle's copies are written by set_weights."""
+    from nova_winograd.ops import check, get_lib
+
+    lib = get_lib()
+    g = torch.Generator().manual_seed(K * C)
+    B, H = 2, 13
+    x = torch.randn(B, C, H, H, generator=g).half().to(DEV)
+    w = torch.randn(K, C, 3, 3, generator=g).to(DEV) * 0.05
+    outs = {}
+    for path in (1, 3, 5, 6, 7):
+        h = lib.nova_create()
+        try:
+            lib.nova_set_path(h, path)
+            for scale in (2.0, 1.0):
+                ws = w * scale
+                lib.nova_set_weights(h, ws.data_ptr(), K, C)
+                check()
+                y = torch.empty(B, K, H, H, dtype=torch.float16, device=DEV)
+                lib.nova_forward(h, x.data_ptr(), y.data_ptr(), B, H, H, 1)
+                lib.nova_get_last_error()
+                torch.cuda.synchronize()
+            outs[path] = (lib.nova_get_last_path(h), y)
+        finally:
+            lib.nova_destroy(h)
+    for path, (ran, y) in outs.items():
+        print(f"[filter copies] K={K} C={C} asked {path} ran {ran}", flush=True)
+        if ran in (6, 7):
+            assert torch.equal(y, outs[1][1])
+        elif ran in (3, 5):  # another order of the channel sums
+            d = (y.float() - outs[1][1].float()).norm() / outs[1][1].float().norm()
+            assert d <= 5e-3
+    if outs[3][0] == 3 and outs[5][0] == 5:
+        assert torch.equal(outs[3][1], outs[5][1])

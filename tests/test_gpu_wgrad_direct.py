@@ -107,3 +107,41 @@ def test_infinities_stay_in_their_channels(W):
     keep = torch.arange(K, device=DEV) != 3
     assert torch.equal(got[keep], base[keep])
     assert not torch.isfinite(got[3, :, 0, 0]).any()
+
+
+@pytest.mark.parametrize("B,C,K,H,W,pad,f32", [
+    (3, 33, 31, 7, 7, 1, False), (2, 70, 65, 28, 28, 1, False), (4, 16, 40, 56, 56, 0, False),
+    (2, 3, 70, 9, 12, 2, False), (1, 320, 64, 16, 16, 1, False), (2, 8, 9, 10, 10, 1, True),
+    (0, 4, 5, 8, 8, 1, False)])
+def test_bias_gradient(B, C, K, H, W, pad, f32):
+    """nova_weight_bias_grad: the same filter gradient, and the channel sums of
+    dY: sums over n = B*Ho*Wo terms, each addition within 2^-24 of its result;
+    no chain is longer than n / 8 (8 waves or more share a channel's pixels)
+    plus the 8 waves and at most 256 splits."""
+    from nova_winograd.ops import check, get_lib
+
+    print(f"[bias grad] B={B} C={C} K={K} H={H} W={W} pad={pad} f32={f32}", flush=True)
+    lib = get_lib()
+    g = torch.Generator().manual_seed(B + K)
+    Ho, Wo = H + 2 * pad - 2, W + 2 * pad - 2
+    x = torch.randn(B, C, H, W, generator=g).half().to(DEV)
+    dy = torch.randn(B, K, Ho, Wo, generator=g).to(DEV) * 0.01
+    dy = dy if f32 else dy.half()
+    gw = torch.full((K, C, 3, 3), float("nan"), device=DEV)
+    gb = torch.full((K,), float("nan"), device=DEV)
+    alone = torch.empty_like(gw)
+    h = lib.nova_create()
+    try:
+        args = (B, C, K, H, W, pad, 1 if f32 else 0)
+        lib.nova_weight_bias_grad(h, x.data_ptr(), dy.data_ptr(), gw.data_ptr(), gb.data_ptr(),
+                                  *args)
+        check()
+        lib.nova_weight_grad(h, x.data_ptr(), dy.data_ptr(), alone.data_ptr(), *args)
+        check()
+        torch.cuda.synchronize()
+    finally:
+        lib.nova_destroy(h)
+    assert torch.equal(gw, alone)
+    want = dy.double().sum(dim=(0, 2, 3))
+    bound = (B * Ho * Wo / 8 + 264) * 2.0**-24 * dy.double().abs().sum(dim=(0, 2, 3))
+    assert ((gb.double() - want).abs() <= bound).all()
