@@ -179,7 +179,7 @@ hipError_t launch_wgemm(const uint16_t* U, const uint16_t* V, uint16_t* M, int K
 // (ResNet-50 at batch 32: 128@28^2 31.7 -> 28.9 us, 256@14^2 31.2 -> 30.3,
 // 512@7^2 29.0 -> 28.4) and costs when V is re-read more often (320@128^2 at
 // batch 1, five reads: 43.1 -> 45.1 us; 640@64^2, ten: 36.7 -> 39.1 us).
-int wgemm_v_reads(int K, int BP);
+int wgemm_v_reads(int K, int Cp, int BP);
 // Kernel name (template configuration) launch_wgemm picks for this shape.
 const char* wgemm_name(int K, int Cp, int BP);
 // GEMV-like shapes (BP <= 32, or 48 above K = 1024; U block copy under

@@ -101,6 +101,29 @@ __device__ __forceinline__ unsigned add_residual2(unsigned h2, unsigned r2, int 
            ((unsigned)__builtin_bit_cast(unsigned short, hi) << 16);
 }
 
+// 16 bytes per lane from a buffer resource straight into LDS: lane l's bytes
+// land at dst + 16*l (dst wave-uniform), zeros where the offset is out of
+// range. The address must be a multiple of 4. Counted in vmcnt.
+__device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t r, void* dst, int off,
+                                           int soff) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16,
+                                             off, soff, 0, 0);
+}
+
+// Waits until at most N of the wave's vector memory operations are in flight.
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+    __builtin_amdgcn_s_waitcnt((N & 15) | (N >> 4 << 14) | (7 << 4) | (15 << 8));
+}
+
+// Workgroup barrier: LDS accesses before it are over after it. Unlike
+// __syncthreads it leaves direct loads and stores in flight.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 // Workgroups are dispatched round-robin over the 8 XCDs, each with its own
 // L2. This bijection maps the dispatch index L (0..N-1) to a work index such
 // that every XCD receives one contiguous range of work items, so spatial

@@ -14,6 +14,7 @@
 // multiple of 8 and zero padded, so partial 32-channel steps only mask whole
 // 8-channel groups. No atomics, no split-K: results are deterministic.
 // Byte offsets are 32-bit: U, V and M must each stay below 2 GB.
+#include <algorithm>
 #include <type_traits>
 
 #include "nova_internal.h"
@@ -25,6 +26,7 @@ typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef unsigned int v2u __attribute__((ext_vector_type(2)));
+typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 
 constexpr int kOob = (int)0x80000000;  // byte offset past every buffer: loads 0, stores dropped
 
@@ -144,40 +146,61 @@ static hipError_t launch_cfg(const uint16_t* U, const uint16_t* V, uint16_t* M, 
 
 // ---------------------------------------------------------------------------
 // LDS-tiled variant for larger shapes. Workgroup tile = TK output channels x
-// TB tiles (bp) of one position, WK x WB waves, channels in stages of 64
-// (two MFMA k-steps): every stage is copied global -> registers -> LDS with
-// 16-byte loads (one 128-byte line per row when Cp >= 64), double buffered so
-// the next stage's loads are in flight while the current one is multiplied.
-// LDS rows are 128 bytes with an XOR swizzle of their 16-byte chunks (see
-// the kernel), conflict-free for both the staging writes and the fragment
-// reads.
+// TB tiles (bp) of one position, WK x WB waves, channels in stages of 64 (two
+// MFMA k-steps, one 128-byte line per row when Cp >= 64). Stages go from
+// memory to LDS directly (no registers in between), NST buffers, NST - 1
+// stages ahead of the one that is multiplied. The buffers are separate arrays,
+// each named by its own code: the compiler tells them apart and does not wait
+// for a direct load into one before a read of another (with one array it
+// waits for every load in flight, which is what made an earlier version of
+// this slower than staging through registers).
+//
+// LDS rows are 128 bytes, 16-byte chunk c of row r at c ^ ((r >> 1) & 7):
+// conflict-free on the 64 banks for the fragment reads (16 lanes on 16
+// consecutive rows, one chunk each); a direct load writes 64 consecutive
+// chunks, so its lanes fetch the permuted chunks of 8 rows' lines.
+//
+// What bounds it: L2 -> CU traffic, 2 * 64 * (nkt * BP + nbt * K) * Cp bytes
+// (nkt, nbt: tiles along K and BP), at 7-10 TB/s, and the latency of a stage.
+// Measured on MI355X (launch in a forward, us, 64-row tiles staged through
+// registers -> this kernel with the rule's tile): 320@64^2 batch 16 62.6 ->
+// 51.2 (64 x 128, 606 MB of traffic -> 160 x 128, 368 MB), batch 8 33.2 ->
+// 27.2; 1280 -> 640@32^2 batch 2 32.4 -> 27.6; 1280@32^2 batch 4 78.8 -> 64.5;
+// ResNet-50 batch 32 256@14^2 6.7 -> 6.2, 512@7^2 9.3 -> 8.9.
 // ---------------------------------------------------------------------------
 constexpr int kStageC = 64;
 
-template <int TK, int TB, int WK, int WB, int PF, int SM>
+// A 16-byte store with a scalar offset. The data registers stay live over two
+// wait states: written by the instruction right behind the store, they reach
+// memory with the new value in the last lanes of each 16 (seen on gfx950; the
+// compiler separates such pairs only for stores without a scalar offset).
+__device__ __forceinline__ void store_b128(v4u v, __amdgpu_buffer_rsrc_t r, int off, int soff,
+                                           bool write_through) {
+    if (write_through)
+        __builtin_amdgcn_raw_buffer_store_b128(v, r, off, soff, kWT);
+    else
+        __builtin_amdgcn_raw_buffer_store_b128(v, r, off, soff, 0);
+    asm volatile("s_nop 1" ::"v"(v) : "memory");
+}
+
+template <int TK, int TB, int WK, int WB, int NST, int SM>
 __global__ __launch_bounds__(64 * WK * WB) void wgemm_lds_kernel(const _Float16* __restrict__ U,
                                                         const _Float16* __restrict__ V,
                                                         _Float16* __restrict__ M, int K, int Cp,
                                                         int BP, int nwg) {
-    constexpr int kThreads = 64 * WK * WB;
+    constexpr int kWaves = WK * WB, kThreads = 64 * kWaves;
     constexpr int MT = TK / WK / 16;  // 16x16 tiles per wave along k
     constexpr int NT = TB / WB / 16;  // along bp
-    constexpr int kChunksU = TK * kStageC / 8;  // 16-byte chunks per stage
-    constexpr int kChunksV = TB * kStageC / 8;
-    constexpr int kPerThreadU = (kChunksU + kThreads - 1) / kThreads;
-    constexpr int kPerThreadV = (kChunksV + kThreads - 1) / kThreads;
-    // Double-buffered stages, U then V: rows of kStageC channels (128 bytes),
-    // 16-byte chunk c of row r stored at chunk c ^ ((r >> 1) & 7). The XOR
-    // swizzle keeps both access patterns conflict-free on the 64 banks: the
-    // staging writes (8 lanes per row, two rows per 16 lanes) and the
-    // fragment reads (16 lanes on 16 consecutive rows, one chunk each).
-    __shared__ __align__(16) _Float16 smem[2 * (TK + TB) * kStageC];
-    auto sU = [&](int buf) { return smem + buf * TK * kStageC; };
-    auto sV = [&](int buf) { return smem + 2 * TK * kStageC + buf * TB * kStageC; };
+    constexpr int kBlkU = TK / 8, kBlkV = TB / 8;  // 1 KB blocks (8 rows) of a stage
+    constexpr int kLoads = (kBlkU + kBlkV + kWaves - 1) / kWaves;  // per wave and stage
+    constexpr int kBuf = kLoads * kWaves * 512;  // halves; blocks past the stage hold zeros
+    __shared__ __align__(1024) _Float16 b0[kBuf];
+    __shared__ __align__(1024) _Float16 b1[kBuf];
+    __shared__ __align__(1024) _Float16 b2[NST > 2 ? kBuf : 8];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wk = wave % WK, wb = wave / WK;
     // One-dimensional grid, XCD-aware: every XCD takes a contiguous run of
     // (position, k-tile, bp-tile) items with the bp tile fastest, so all
@@ -190,58 +213,33 @@ __global__ __launch_bounds__(64 * WK * WB) void wgemm_lds_kernel(const _Float16*
     const int n0 = (rem % nbt) * TB;
     const int r16 = lane & 15, g = lane >> 4;
 
-    const __amdgpu_buffer_rsrc_t urs = make_rsrc(U, 2 * (int64_t)64 * K * Cp);
-    const __amdgpu_buffer_rsrc_t vrs = make_rsrc(V, 2 * (int64_t)64 * BP * Cp);
+    const __amdgpu_buffer_rsrc_t urs = make_rsrc(U + (int64_t)p * K * Cp, 2 * (int64_t)K * Cp);
+    const __amdgpu_buffer_rsrc_t vrs = make_rsrc(V + (int64_t)p * BP * Cp, 2 * (int64_t)BP * Cp);
     const __amdgpu_buffer_rsrc_t mrs = make_rsrc(M, 2 * (int64_t)64 * BP * K);
-    const int au = 2 * p * K * Cp;  // uniform byte offsets of position p
-    const int bu = 2 * p * BP * Cp;
 
-    // staging assignment: chunk id -> (row, 8-channel group); 8 chunks per row
-    int uoff[kPerThreadU], ulds[kPerThreadU], voff[kPerThreadV], vlds[kPerThreadV];
+    // load j of the wave: block 8 rows x 8 chunks, lane = (row, slot)
+    int off[kLoads], chan[kLoads];
 #pragma unroll
-    for (int j = 0; j < kPerThreadU; j++) {
-        const int ch = tid + j * kThreads;
-        const int row = ch >> 3, cg = ch & 7;
-        const bool ok = ch < kChunksU && k0 + row < K;
-        uoff[j] = ok ? 2 * ((k0 + row) * Cp + cg * 8) : kOob;
-        ulds[j] = ch < kChunksU ? row * kStageC + (cg ^ ((row >> 1) & 7)) * 8 : -1;
-    }
-#pragma unroll
-    for (int j = 0; j < kPerThreadV; j++) {
-        const int ch = tid + j * kThreads;
-        const int row = ch >> 3, cg = ch & 7;
-        const bool ok = ch < kChunksV && n0 + row < BP;
-        voff[j] = ok ? 2 * ((n0 + row) * Cp + cg * 8) : kOob;
-        vlds[j] = ch < kChunksV ? row * kStageC + (cg ^ ((row >> 1) & 7)) * 8 : -1;
+    for (int j = 0; j < kLoads; j++) {
+        const int blk = j * kWaves + wave;
+        const bool u = blk < kBlkU;
+        const int row = (u ? blk : blk - kBlkU) * 8 + (lane >> 3);
+        chan[j] = 8 * ((lane & 7) ^ ((row >> 1) & 7));
+        const int at = (u ? k0 : n0) + row;
+        const bool ok = u ? at < K : blk < kBlkU + kBlkV && at < BP;
+        off[j] = ok ? 2 * (at * Cp + chan[j]) : kOob;
     }
     const int nstages = (Cp + kStageC - 1) / kStageC;
-    // PF stages in flight in registers: slot st % PF holds stage st from its
-    // load until its copy into LDS
-    h8 ru[PF][kPerThreadU], rv[PF][kPerThreadV];
-    auto gload = [&](int st, h8 (&u)[kPerThreadU], h8 (&v)[kPerThreadV]) {
+    // stage st into buf; stages past the last one load zeros (NST > 2 counts
+    // every stage's loads)
+    auto issue = [&](int st, _Float16* buf) {
         const int c = st * kStageC;
 #pragma unroll
-        for (int j = 0; j < kPerThreadU; j++) {
-            const int cg = (tid + j * kThreads) & 7;
-            const bool cok = c + cg * 8 < Cp;
-            u[j] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(
-                                              urs, cok ? uoff[j] : kOob, au + 2 * c, 0));
+        for (int j = 0; j < kLoads; j++) {
+            const int blk = j * kWaves + wave;
+            load_lds16(blk < kBlkU ? urs : vrs, buf + blk * 512,
+                       c + chan[j] < Cp ? off[j] : kOob, 2 * c);
         }
-#pragma unroll
-        for (int j = 0; j < kPerThreadV; j++) {
-            const int cg = (tid + j * kThreads) & 7;
-            const bool cok = c + cg * 8 < Cp;
-            v[j] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(
-                                              vrs, cok ? voff[j] : kOob, bu + 2 * c, 0));
-        }
-    };
-    auto lstore = [&](int buf, const h8 (&u)[kPerThreadU], const h8 (&v)[kPerThreadV]) {
-#pragma unroll
-        for (int j = 0; j < kPerThreadU; j++)
-            if (ulds[j] >= 0) *reinterpret_cast<h8*>(sU(buf) + ulds[j]) = u[j];
-#pragma unroll
-        for (int j = 0; j < kPerThreadV; j++)
-            if (vlds[j] >= 0) *reinterpret_cast<h8*>(sV(buf) + vlds[j]) = v[j];
     };
 
     f4 acc[MT][NT];
@@ -249,78 +247,91 @@ __global__ __launch_bounds__(64 * WK * WB) void wgemm_lds_kernel(const _Float16*
     for (int mi = 0; mi < MT; mi++)
 #pragma unroll
         for (int ni = 0; ni < NT; ni++) acc[mi][ni] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-
+    // lane (row r16 of each 16-row tile, chunk 4*kk + g); every tile starts at
+    // a multiple of 16 rows, so the swizzle depends on r16
+    const int c0 = g ^ ((r16 >> 1) & 7);
+    auto multiply = [&](const _Float16* buf) {
+        const _Float16* su = buf + (wk * MT * 16 + r16) * kStageC;
+        const _Float16* sv = buf + (TK + wb * NT * 16 + r16) * kStageC;
 #pragma unroll
-    for (int j = 0; j < PF; j++)
-        if (j < nstages) gload(j, ru[j], rv[j]);
-    lstore(0, ru[0], rv[0]);
-    __syncthreads();
-    for (int st0 = 0; st0 < nstages; st0 += PF) {
+        for (int kk = 0; kk < kStageC / 32; kk++) {
+            const int co = (c0 ^ (4 * kk)) * 8;
+            h8 a[MT], b[NT];
 #pragma unroll
-        for (int j = 0; j < PF; j++) {
-            const int st = st0 + j;
-            if (st >= nstages) break;
-            const int buf = st & 1;
-            if (st + PF < nstages) gload(st + PF, ru[j], rv[j]);
-            // lane (row r16 of each 16-row tile, chunk 4*kk + g); every tile
-            // starts at a multiple of 16 rows, so the swizzle depends on r16
-            const int c0 = g ^ ((r16 >> 1) & 7);
-            const _Float16* su = sU(buf) + (wk * MT * 16 + r16) * kStageC;
-            const _Float16* sv = sV(buf) + (wb * NT * 16 + r16) * kStageC;
+            for (int ni = 0; ni < NT; ni++)
+                b[ni] = *reinterpret_cast<const h8*>(sv + ni * 16 * kStageC + co);
 #pragma unroll
-            for (int kk = 0; kk < kStageC / 32; kk++) {
-                const int co = (c0 ^ (4 * kk)) * 8;
-                h8 a[MT], b[NT];
-#pragma unroll
-                for (int mi = 0; mi < MT; mi++)
-                    a[mi] = *reinterpret_cast<const h8*>(su + mi * 16 * kStageC + co);
-#pragma unroll
-                for (int ni = 0; ni < NT; ni++)
-                    b[ni] = *reinterpret_cast<const h8*>(sv + ni * 16 * kStageC + co);
-#pragma unroll
-                for (int mi = 0; mi < MT; mi++)
-#pragma unroll
-                    for (int ni = 0; ni < NT; ni++)
-                        acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[mi], b[ni],
-                                                                             acc[mi][ni], 0, 0, 0);
-            }
-            if (st + 1 < nstages) lstore(buf ^ 1, ru[(j + 1) % PF], rv[(j + 1) % PF]);
-            __syncthreads();
-        }
-    }
-
-    const int mu = 2 * p * BP * K;
-    if constexpr (SM != 0) {
-        // SM 1/2: the M tile goes through LDS as [bp][k] rows and leaves as
-        // whole rows, 16 bytes per lane (SM 2: written through the L2, sc1);
-        // the L2 then holds whole lines instead of 32-byte pieces of 16.
-        if ((K & 7) == 0) {
-            constexpr int kMP = TK + 8;  // halves per staged row
-            static_assert(TB * kMP <= 2 * (TK + TB) * kStageC, "M tile fits in the stages");
-            _Float16* sm = smem;
+            for (int mi = 0; mi < MT; mi++)
+                a[mi] = *reinterpret_cast<const h8*>(su + mi * 16 * kStageC + co);
 #pragma unroll
             for (int mi = 0; mi < MT; mi++)
 #pragma unroll
-                for (int ni = 0; ni < NT; ni++) {
-                    const int bpl = (wb * NT + ni) * 16 + r16;
-                    const int kl = (wk * MT + mi) * 16 + 4 * g;
-                    *reinterpret_cast<h4*>(sm + bpl * kMP + kl) =
-                        h4{(_Float16)acc[mi][ni][0], (_Float16)acc[mi][ni][1],
-                           (_Float16)acc[mi][ni][2], (_Float16)acc[mi][ni][3]};
-                }
-            __syncthreads();
-            typedef unsigned u4 __attribute__((ext_vector_type(4)));
-            constexpr int kCh = TK / 8;  // 16-byte chunks per row
-#pragma unroll
-            for (int e = tid; e < TB * kCh; e += kThreads) {
-                const int row = e / kCh, ch = e % kCh;
-                const int bp = n0 + row, k = k0 + 8 * ch;
-                const u4 v = *reinterpret_cast<const u4*>(sm + row * kMP + 8 * ch);
-                __builtin_amdgcn_raw_buffer_store_b128(
-                    v, mrs, (bp < BP && k < K) ? 2 * (bp * K + k) : kOob, mu, SM == 2 ? kWT : 0);
-            }
-            return;
+                for (int ni = 0; ni < NT; ni++)
+                    acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[mi], b[ni],
+                                                                         acc[mi][ni], 0, 0, 0);
         }
+    };
+    // stage st's loads are over (the next NST - 2 stages' may be in flight);
+    // the barrier also ends stage st - 1's products, whose buffer is loaded
+    auto turn = [&](int st, const _Float16* cur, _Float16* next) {
+        wait_vmcnt<kLoads * (NST - 2)>();
+        lds_barrier();
+        if (NST > 2 || st + 1 < nstages) issue(st + NST - 1, next);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(cur);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    issue(0, b0);
+    if constexpr (NST > 2) issue(1, b1);
+    for (int st = 0; st < nstages; st += NST) {
+        if constexpr (NST == 2) {
+            turn(st, b0, b1);
+            if (st + 1 < nstages) turn(st + 1, b1, b0);
+        } else {
+            turn(st, b0, b2);
+            if (st + 1 < nstages) turn(st + 1, b1, b0);
+            if (st + 2 < nstages) turn(st + 2, b2, b1);
+        }
+    }
+    wait_vmcnt<0>();
+    lds_barrier();
+
+    const int mu = 2 * p * BP * K;
+    // The M tile goes through LDS as [bp][k] rows, half of them in each
+    // buffer, and leaves as whole rows, 16 bytes per lane (SM 2: written
+    // through the L2, sc1); the L2 then holds whole lines instead of 32-byte
+    // pieces of 16.
+    if ((K & 7) == 0) {
+        constexpr int kMP = TK + 8;    // halves per staged row
+        constexpr int kRows = TB / 2;  // rows per buffer
+        static_assert(kRows % 16 == 0 && kRows * kMP <= kBuf, "M tile fits in the stages");
+#pragma unroll
+        for (int mi = 0; mi < MT; mi++)
+#pragma unroll
+            for (int ni = 0; ni < NT; ni++) {
+                const int bpl = (wb * NT + ni) * 16;  // uniform
+                const int kl = (wk * MT + mi) * 16 + 4 * g;
+                const h4 v = h4{(_Float16)acc[mi][ni][0], (_Float16)acc[mi][ni][1],
+                                (_Float16)acc[mi][ni][2], (_Float16)acc[mi][ni][3]};
+                if (bpl < kRows)
+                    *reinterpret_cast<h4*>(b0 + (bpl + r16) * kMP + kl) = v;
+                else
+                    *reinterpret_cast<h4*>(b1 + (bpl - kRows + r16) * kMP + kl) = v;
+            }
+        lds_barrier();
+        constexpr int kCh = TK / 8;  // 16-byte chunks per row
+        auto rows_out = [&](const _Float16* buf, int bp0) {
+#pragma unroll
+            for (int e = tid; e < kRows * kCh; e += kThreads) {
+                const int row = e / kCh, ch = e % kCh;
+                const int bp = bp0 + row, k = k0 + 8 * ch;
+                store_b128(*reinterpret_cast<const v4u*>(buf + row * kMP + 8 * ch), mrs,
+                           (bp < BP && k < K) ? 2 * (bp * K + k) : kOob, mu, SM == 2);
+            }
+        };
+        rows_out(b0, n0);
+        rows_out(b1, n0 + kRows);
+        return;
     }
     const bool vec_store = (K & 3) == 0;
 #pragma unroll
@@ -363,7 +374,7 @@ static int m_epilogue(int K, int BP) {
     return m_bytes <= ((int64_t)32 << 20) ? 2 : 1;
 }
 
-template <int TK, int TB, int WK, int WB, int PF>
+template <int TK, int TB, int WK, int WB, int NST>
 static hipError_t launch_lds(const uint16_t* U, const uint16_t* V, uint16_t* M, int K, int Cp,
                              int BP, hipStream_t s) {
     const unsigned grid = 64u * (unsigned)((BP + TB - 1) / TB) * (unsigned)((K + TK - 1) / TK);
@@ -372,9 +383,9 @@ static hipError_t launch_lds(const uint16_t* U, const uint16_t* V, uint16_t* M, 
                reinterpret_cast<const _Float16*>(V), reinterpret_cast<_Float16*>(M), K, Cp, BP);
     };
     if (m_epilogue(K, BP) == 2)
-        go(wgemm_lds_kernel<TK, TB, WK, WB, PF, 2>);
+        go(wgemm_lds_kernel<TK, TB, WK, WB, NST, 2>);
     else
-        go(wgemm_lds_kernel<TK, TB, WK, WB, PF, 1>);
+        go(wgemm_lds_kernel<TK, TB, WK, WB, NST, 1>);
     return hipGetLastError();
 }
 
@@ -535,78 +546,112 @@ const char* wgemm_blocks_name(int BP) {
 // per wave, which halves the V fragment loads and doubles the U bytes each
 // wave keeps in flight: 512@7^2 at batch 1 7.1 -> 6.5 us, 1280@8^2 at batch
 // 2 39.2 -> 34.9 us); LDS-tiled otherwise, the tile chosen from a sweep of
-// every tile shape on MI355X
-// (GEMM launch alone, per-kernel events, min of 2 x 60 launches, us; the
-// results are bit-identical across tile shapes):
-//  * 128 x 128 for K >= 512 with BP >= 256 (512@7^2 B=64 17.1 vs 20.3-22.4
-//    for the other shapes, B=128 31.4 vs 35.1-41.4);
-//  * 128 x 64 (8 waves) for K >= 1024 below 128 tiles (1280@16^2 B=2 33.6 vs
-//    36.4 for 64 x 64; 1280@32^2 B=1 34.0 vs 35.9; 640->1280@16^2 B=2 17.8 vs
-//    19.5);
-//  * 64 x 128, two stages in flight, for larger work: K >= 640 from 64 tiles,
-//    K >= 512 from 128, K >= 256 from 200, K <= 128 from 1600 (ResNet-50
-//    256@14^2 B=32 9.5 vs 11.0, B=128 24.6 vs 29.1; 512@7^2 B=32 10.8 vs
-//    11.2 for 128 x 128; 128@28^2 B=128 23.0 vs 26.0; SD-1.5 640@32^2 B=2
-//    14.4 vs 15.6, 320@64^2 B=2 8.8 vs 9.7; SDXL 640@64^2 14.5 vs 17.7;
-//    1280->640@32^2 B=2 23.6 vs 30.4). A second sweep (back-to-back launches
-//    of the GEMM alone) favoured it for K <= 128 from 200 tiles as well
-//    (128@28^2 B=32 7.17 -> 6.38), but inside forwards, with V just written,
-//    it lost there (batch 32 8.95 -> 9.41 us per GEMM), so 64 x 64 stays;
-//  * 64 x 96 with four waves and one stage in flight where that tile width
-//    fills its last tile 15 points better than 128 (GEMM alone, us:
-//    256@14^2 B=32, 288 tiles, 6.98 -> 6.39; 640@32^2 B=2, 72 tiles, 13.9 ->
-//    12.4, with 320 -> 640 channels 7.9 -> 7.3, 1280 -> 640 24.0 -> 21.2;
-//    640@32^2 B=4 21.3 -> 19.9; inside forwards 640@32^2 B=2 13.2 -> 11.9,
-//    whole forward 30.0 -> 28.5; 256@14^2 B=32 unchanged, 9.1 vs 9.0); where
-//    the fills are close 64 x 128 stays ahead (256@14^2 B=64 12.5 vs 12.4,
-//    128@28^2 B=64 11.9 vs 12.4);
-//  * else 64 x 64: two stages in flight from 128 tiles (128@28^2 B=32 8.7,
-//    128 x 128 8.7, 64 x 128 8.9; 256@14^2 B=16 7.5 vs 8.1 for 64 x 128),
-//    8 waves up to K = 256, 4 waves beyond (512@7^2 B=8 7.7 vs 8.0 with 8
-//    waves and 9.0 with 64 x 128; B=16 8.0 vs 9.3).
-// Share of a row of bp tiles of width tb that holds real tiles.
-static double bp_fill(int BP, int tb) { return (double)BP / (tb * ((BP + tb - 1) / tb)); }
+// every tile shape on MI355X (GEMM launches inside forwards, per-kernel
+// events, us; the results are bit-identical across tile shapes). Tiles that
+// leave no more of K empty than 64-row ones, as large as the work allows:
+//  * 160 x 128 where 160 divides K as well as 64 does, from 240 tiles (128
+//    above K = 1024): fewer and larger workgroups read V and U less often
+//    (320@64^2 B=16 60.3 for 64 x 128, 59.5 for 128 x 128, 51.0; B=8 33.4,
+//    31.5, 27.4; 640@64^2 B=8 91.1, 81.8, 73.3; 160@28^2 B=32 13.1, 11.7,
+//    10.4; 1280@32^2 B=4, 144 tiles, 76.5 for 64 x 96, 72.1, 66.6); below
+//    that the grid is too small (640@64^2 B=1, 121 tiles: 14.6 against 13.6);
+//  * the same tile with three buffers for deep layers at 64 to 128 tiles (U
+//    streams from memory, one workgroup per CU: 1280 -> 640@32^2 B=2 27.6
+//    against 30.2 with two buffers and 32.1 for 64 x 96; 640@64^2 B=1 12.3
+//    against 13.6), below 1024 channels only where 96-tile widths do not fit
+//    BP better (640@32^2 B=2, 72 tiles, 11.7 against 11.4; with 320 channels
+//    8.7 against 7.6);
+//  * 96 x 96 or 96 x 128 where 96 divides K as well, from 128 tiles (whole
+//    forwards, eager, us: 384@20^2 B=12 24.9 for 64 x 64, 21.9; 480@30^2 B=6
+//    31.9, 30.0; 192@28^2 B=32 34.4 for 64 x 128, 96 x 128 34.5, 96 x 96 33.5;
+//    launch alone 96@56^2 B=16 12.7 for 64 x 128, 96 x 96 10.7, 96 x 128 9.7;
+//    384@28^2 B=8 9.0, 9.5, 8.2), the width that fills BP better;
+//  * 128 rows where 128 divides K as well: 128 x 192 from 500 tiles that it
+//    fills (256@14^2 B=64 27.2 -> 26.4, B=128 54.0 -> 51.6 for whole
+//    forwards), 128 x 128 from 300 (48 -> 200@21^2 B=20 19.0 -> 18.1), for
+//    K >= 512 from 256 (512@7^2 B=64 13.9 vs 15.5-17.3 for the other shapes,
+//    B=128 24.9 vs 26.2-30.8), for K of 97 to 128 from 1600 (128@28^2 B=64
+//    10.7 for 64 x 128, 10.2, B=128 25.4, 22.8);
+//  * 128 x 64 (8 waves) for K >= 1024 below 128 tiles (a register-staged
+//    form: 1280@16^2 B=2 33.6 vs 36.4 for 64 x 64; 1280@32^2 B=1 34.0 vs
+//    35.9; 640->1280@16^2 B=2 17.8 vs 19.5);
+//  * 64 x 128 for larger work: K >= 640 from 64 tiles, K >= 512 from 128,
+//    K >= 256 from 200 (512@7^2 B=32 9.0 vs 10.0 for 128 x 128; 256@14^2 B=24
+//    18.7 vs 19.0);
+//  * 64 x 96 with four waves where that tile width fills its last tile 15
+//    points better than 128, for K >= 256 from 128 tiles (256@14^2 B=32, 288
+//    tiles, 6.6 against 7.5, B=16 16.3 -> 15.9 for a forward; 640@32^2 B=2, 72
+//    tiles, 11.4 against 12.4);
+//  * else 64 x 64: four waves above K = 256 or from 128 tiles and four stages
+//    (512@7^2 B=16 7.8 against 8.0), else eight (with one or two stages four
+//    lost 1.5-4 % of a forward: 48 -> 200@21^2 B=20, 128@56^2 B=2). Odd
+//    channel counts (K % 8 != 0, M stored in pieces) stay with 64 rows
+//    (189@15^2 B=45 28.5 against 30.0 for 96 x 128).
+// Share of a row of tiles of width t that n fills.
+static double fill(int n, int t) { return (double)n / (t * ((n + t - 1) / t)); }
 
-static int wgemm_cfg(int K, int BP) {
+static int wgemm_cfg(int K, int Cp, int BP) {
     if (BP <= 16) return 0;
+    const bool narrow = fill(BP, 96) >= fill(BP, 128) + 0.15;
+    if (K % 8 == 0) {
+        if (K >= 160 && fill(K, 160) >= fill(K, 64)) {
+            if (BP >= 240 || (K >= 1024 && BP >= 128)) return 8;
+            if (K >= 640 && K < 1024 && Cp >= (narrow ? 1024 : 640) && BP >= 64 && BP <= 128)
+                return 9;
+        }
+        if (BP >= 128 && K >= 65 && fill(K, 96) >= std::max(fill(K, 64), fill(K, 128)))
+            return fill(BP, 96) >= fill(BP, 128) + 0.03 ? 11 : 10;
+        if (K >= 192 && fill(K, 128) >= fill(K, 64)) {
+            if (BP >= 500 && fill(BP, 192) >= fill(BP, 128)) return 3;
+            if (BP >= 300) return 2;
+        }
+        if (BP >= 1600 && K > 96 && K <= 128) return 2;
+    }
     if (K >= 512 && BP >= 256) return 2;
     if (K >= 1024 && BP < 128) return 5;
+    if (K >= 256 && BP >= 128 && narrow) return 7;
     if ((K >= 640 && BP >= 64) || (K >= 512 && BP >= 128) || (K >= 256 && BP >= 200) ||
         (K <= 128 && BP >= 1600))
-        return bp_fill(BP, 96) >= bp_fill(BP, 128) + 0.15 ? 7 : 6;
-    if (BP >= 128) return 3;
-    return K <= 256 ? 4 : 1;
+        return narrow ? 7 : 6;
+    return K > 256 || (BP >= 128 && Cp >= 256) ? 1 : 4;
 }
 
-int wgemm_v_reads(int K, int BP) {
-    const int cfg = wgemm_cfg(K, BP);
-    const int tk = (cfg == 2 || cfg == 5) ? 128 : 64;  // output channels per workgroup tile
-    return (K + tk - 1) / tk;
+int wgemm_v_reads(int K, int Cp, int BP) {
+    static const int tk[] = {64, 64, 128, 128, 64, 128, 64, 64, 160, 160, 96, 96};
+    const int t = tk[wgemm_cfg(K, Cp, BP)];  // output channels per workgroup tile
+    return (K + t - 1) / t;
 }
 
 const char* wgemm_name(int K, int Cp, int BP) {
-    (void)Cp;
-    static const char* names[] = {"wgemm_kernel<2, 1, 2, 1, 4>", "wgemm_lds_kernel<64, 64, 2, 2, 1>",
-                                  "wgemm_lds_kernel<128, 128, 2, 4, 1>",
+    static const char* names[] = {"wgemm_kernel<2, 1, 2, 1, 4>", "wgemm_lds_kernel<64, 64, 2, 2, 2>",
+                                  "wgemm_lds_kernel<128, 128, 2, 4, 2>",
+                                  "wgemm_lds_kernel<128, 192, 2, 4, 2>",
                                   "wgemm_lds_kernel<64, 64, 2, 4, 2>",
-                                  "wgemm_lds_kernel<64, 64, 2, 4, 1>",
-                                  "wgemm_lds_kernel<128, 64, 2, 4, 1>",
+                                  "wgemm_lds_kernel<128, 64, 2, 4, 2>",
                                   "wgemm_lds_kernel<64, 128, 2, 4, 2>",
-                                  "wgemm_lds_kernel<64, 96, 2, 2, 1>"};
-    return names[wgemm_cfg(K, BP)];
+                                  "wgemm_lds_kernel<64, 96, 2, 2, 2>",
+                                  "wgemm_lds_kernel<160, 128, 2, 4, 2>",
+                                  "wgemm_lds_kernel<160, 128, 2, 4, 3>",
+                                  "wgemm_lds_kernel<96, 128, 2, 4, 2>",
+                                  "wgemm_lds_kernel<96, 96, 2, 2, 2>"};
+    return names[wgemm_cfg(K, Cp, BP)];
 }
 
 hipError_t launch_wgemm(const uint16_t* U, const uint16_t* V, uint16_t* M, int K, int Cp,
                         int BP, hipStream_t s) {
-    switch (wgemm_cfg(K, BP)) {
+    switch (wgemm_cfg(K, Cp, BP)) {
         case 0: return launch_cfg<2, 1, 2, 1, 4>(U, V, M, K, Cp, BP, s);
-        case 1: return launch_lds<64, 64, 2, 2, 1>(U, V, M, K, Cp, BP, s);
-        case 2: return launch_lds<128, 128, 2, 4, 1>(U, V, M, K, Cp, BP, s);
-        case 3: return launch_lds<64, 64, 2, 4, 2>(U, V, M, K, Cp, BP, s);
-        case 5: return launch_lds<128, 64, 2, 4, 1>(U, V, M, K, Cp, BP, s);
+        case 1: return launch_lds<64, 64, 2, 2, 2>(U, V, M, K, Cp, BP, s);
+        case 2: return launch_lds<128, 128, 2, 4, 2>(U, V, M, K, Cp, BP, s);
+        case 3: return launch_lds<128, 192, 2, 4, 2>(U, V, M, K, Cp, BP, s);
+        case 5: return launch_lds<128, 64, 2, 4, 2>(U, V, M, K, Cp, BP, s);
         case 6: return launch_lds<64, 128, 2, 4, 2>(U, V, M, K, Cp, BP, s);
-        case 7: return launch_lds<64, 96, 2, 2, 1>(U, V, M, K, Cp, BP, s);
-        default: return launch_lds<64, 64, 2, 4, 1>(U, V, M, K, Cp, BP, s);
+        case 7: return launch_lds<64, 96, 2, 2, 2>(U, V, M, K, Cp, BP, s);
+        case 8: return launch_lds<160, 128, 2, 4, 2>(U, V, M, K, Cp, BP, s);
+        case 9: return launch_lds<160, 128, 2, 4, 3>(U, V, M, K, Cp, BP, s);
+        case 10: return launch_lds<96, 128, 2, 4, 2>(U, V, M, K, Cp, BP, s);
+        case 11: return launch_lds<96, 96, 2, 2, 2>(U, V, M, K, Cp, BP, s);
+        default: return launch_lds<64, 64, 2, 4, 2>(U, V, M, K, Cp, BP, s);
     }
 }
 

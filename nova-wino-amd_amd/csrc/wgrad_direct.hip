@@ -205,8 +205,7 @@ __global__ __launch_bounds__(kThreads) void wgrad_direct_kernel(WdArgs a) {
                 se[s] = __builtin_amdgcn_raw_buffer_load_b32(rs, o + 16, so & ~3, 0);
             } else {
                 char* dst = s < nslot ? buf + (blk0 + s * nwav) * 1024 : spare;
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                    rs, (__attribute__((address_space(3))) void*)dst, 16, o, so, 0, 0);
+                load_lds16(rs, dst, o, so);
             }
         };
         if (check) {
@@ -350,15 +349,6 @@ __global__ __launch_bounds__(kThreads) void wgrad_direct_kernel(WdArgs a) {
         }
         advance(up);
     };
-    // The waves' LDS accesses before it are over after it (reads have been
-    // consumed, writes waited for; a workgroup fence would also wait for the
-    // direct loads still in flight).
-    auto barrier = [&]() {
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-    };
-
     if constexpr (kStage == kRegs) {
         Unit us = ul;
         auto turn = [&](int i, char* cur, char* nxt) {
@@ -370,14 +360,14 @@ __global__ __launch_bounds__(kThreads) void wgrad_direct_kernel(WdArgs a) {
                 store_unit(us, nxt);
                 advance(us);
             }
-            barrier();
+            lds_barrier();
         };
         if (nu > 0) {
             load_unit(buf0);
             store_unit(us, buf0);
             advance(us);
         }
-        barrier();
+        lds_barrier();
         for (int i = 0; i < nu; i += 2) {
             turn(i, buf0, buf1);
             if (i + 1 < nu) turn(i + 1, buf1, buf0);
@@ -391,10 +381,10 @@ __global__ __launch_bounds__(kThreads) void wgrad_direct_kernel(WdArgs a) {
         const bool late = wave >= 4;
         auto turn = [&](int i, char* cur, char* nxt2) {
             if (i + 1 < nu)
-                __builtin_amdgcn_s_waitcnt(kSlots | (7 << 4) | (15 << 8));  // vmcnt(kSlots)
+                wait_vmcnt<kSlots>();
             else
-                __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));  // vmcnt(0)
-            barrier();
+                wait_vmcnt<0>();
+            lds_barrier();
             if (!late && i + 2 < nu) load_unit(nxt2);
             __builtin_amdgcn_sched_barrier(0);
             products(cur);
@@ -408,7 +398,7 @@ __global__ __launch_bounds__(kThreads) void wgrad_direct_kernel(WdArgs a) {
             if (i + 1 < nu) turn(i + 1, buf1, buf0);
             if (i + 2 < nu) turn(i + 2, buf2, buf1);
         }
-        barrier();
+        lds_barrier();
     }
 
     // The WP waves' sums, a quarter of every tile at a time (8 output
@@ -422,7 +412,7 @@ __global__ __launch_bounds__(kThreads) void wgrad_direct_kernel(WdArgs a) {
     float* const out = a.out + (int64_t)sp * a.K * a.C * 9;
     if (PAD < 2 && a.bias != nullptr && c0 == 0) {
         if (wc == 0) red[0][wave * 64 + lane] = bunit;
-        barrier();
+        lds_barrier();
         if (tid < 32 * WK && k0 + tid < a.K) {
             const int w0 = tid >> 5;  // the wave with this row, wc = 0 and wp = 0
             float v = 0.0f;
@@ -433,7 +423,7 @@ __global__ __launch_bounds__(kThreads) void wgrad_direct_kernel(WdArgs a) {
             }
             a.bias[(int64_t)sp * a.K + k0 + tid] = v;
         }
-        barrier();
+        lds_barrier();
     }
 #pragma unroll
     for (int q = 0; q < 4; q++) {
@@ -442,7 +432,7 @@ __global__ __launch_bounds__(kThreads) void wgrad_direct_kernel(WdArgs a) {
 #pragma unroll
             for (int e = 0; e < 4; e++)
                 red[t / 3][(t % 3) * kTapPitch + (wave * 4 + e) * 64 + lane] = acc[t][4 * q + e];
-        barrier();
+        lds_barrier();
         for (int i = tid; i < WK * WC * 8 * 288; i += kThreads) {
             // dw row of pair `pair`: 32 input channels x 9 taps
             const int rowi = i / 288, j = i - rowi * 288;
@@ -456,7 +446,7 @@ __global__ __launch_bounds__(kThreads) void wgrad_direct_kernel(WdArgs a) {
             for (int p = 1; p < WP; p++) v += r[o + p * WK * WC * 256];
             if (cc < a.C && kk < a.K) out[((int64_t)kk * a.C + cc) * 9 + tap] = v;
         }
-        barrier();
+        lds_barrier();
     }
 }
 
