@@ -286,7 +286,7 @@ def _grad_input_nova(holder, go, weight, padding, dtype):
     C = weight.shape[1]
     gi = torch.empty(B, C, Ho + 2 * pb - 2, Wo + 2 * pb - 2, dtype=torch.float16,
                      device=go.device)
-    hd.lib.nova_forward(hd.h, ptr(g16), ptr(gi), B, Ho, Wo, pb)
+    hd.lib.nova_forward(hd.h, g16.data_ptr(), gi.data_ptr(), B, Ho, Wo, pb)
     check("backward (grad input)")
     return gi.to(dtype)
 
@@ -322,12 +322,13 @@ def _grad_weight(holder, inp, go, weight, padding, bias=None):
     gw = torch.empty(K, C, 3, 3, dtype=torch.float32, device=go.device)
     f32 = 1 if g.dtype == torch.float32 else 0
     if bias is None:
-        hd.lib.nova_weight_grad(hd.h, ptr(x16), ptr(g), ptr(gw), B, C, K, H, W, padding, f32)
+        hd.lib.nova_weight_grad(hd.h, x16.data_ptr(), g.data_ptr(), gw.data_ptr(), B, C, K, H, W,
+                                padding, f32)
         check("backward (grad weight)")
         return gw.to(weight.dtype)
     gb = torch.empty(K, dtype=torch.float32, device=go.device)
-    hd.lib.nova_weight_bias_grad(hd.h, ptr(x16), ptr(g), ptr(gw), ptr(gb), B, C, K, H, W, padding,
-                                 f32)
+    hd.lib.nova_weight_bias_grad(hd.h, x16.data_ptr(), g.data_ptr(), gw.data_ptr(), gb.data_ptr(),
+                                 B, C, K, H, W, padding, f32)
     check("backward (grad weight and bias)")
     return gw.to(weight.dtype), gb.to(bias.dtype)
 
@@ -512,16 +513,20 @@ class NovaWinogradConv2d(nn.Module):
         if self._handle is None:
             self._handle = _Handle()
         hd = self._handle
-        hd.set_stream(self.weight.device)
-        key = _weight_key(self.weight)
+        weight = self.weight  # one nn.Module lookup
+        hd.set_stream(weight.device)
+        key = _weight_key(weight)
         ref = hd.key
-        if not (ref is not None and ref[0]() is self.weight and ref[1] == key):
-            hd.set_weights(self.weight)
-            hd.key = (weakref.ref(self.weight), key)
-            self._weight_version = self.weight._version
-            self._V_gemm = None
-            self._M_gemm = None
-            self._last_config = None
+        if not (ref is not None and ref[0]() is weight and ref[1] == key):
+            hd.set_weights(weight)
+            hd.key = (weakref.ref(weight), key)
+            self._weight_version = weight._version
+            # the workspace follows the layer's shape and device: new values of
+            # the same parameter (an optimizer step) keep it
+            if ref is None or ref[1][3:] != key[3:]:
+                self._V_gemm = None
+                self._M_gemm = None
+                self._last_config = None
 
     def _ensure_workspace(self, batch, H, W):
         """Allocate the reference-sized workspace when the configuration
