@@ -151,14 +151,14 @@ constexpr int64_t kWTSmallBytes = (int64_t)2 << 20;
 // V store cache policy (results unchanged): the forms whose wave stores are
 // whole 128-byte lines (the tile-block forms in the product layout with at
 // least 64 channels per workgroup and ldv % 64 == 0, and the run form) write
-// through the L2; otherwise stream_v asks for the non-temporal (nt) policy
-// (see wgemm_v_reads for when it pays).
+// through the L2; otherwise stream_v 1 asks for the non-temporal (nt) policy
+// (see wgemm_v_reads for when it pays); stream_v 2 asks for it in every form.
 // vfrag: 0 = V in the product layout V[p][bp][ldv]; otherwise the number of
 // 32-channel chunks of the two-pass layout (1 KB MFMA B-operand blocks of 16
 // tiles x 32 channels; pstride = ceil(BP / 16) * vfrag * 512 halves).
 hipError_t launch_input_transform(const uint16_t* x, uint16_t* V, int B, int C, int H, int W,
                                   int pad, int nh, int nw, int ldv, int64_t pstride,
-                                  hipStream_t s, bool nhwc = false, bool stream_v = false,
+                                  hipStream_t s, bool nhwc = false, int stream_v = 0,
                                   int vfrag = 0);
 
 // ---- output transform ----------------------------------------------------
@@ -180,6 +180,9 @@ hipError_t launch_wgemm(const uint16_t* U, const uint16_t* V, uint16_t* M, int K
 // 512@7^2 29.0 -> 28.4) and costs when V is re-read more often (320@128^2 at
 // batch 1, five reads: 43.1 -> 45.1 us; 640@64^2, ten: 36.7 -> 39.1 us).
 int wgemm_v_reads(int K, int Cp, int BP);
+// A deep layer's GEMM whose U streams past the caches (three-buffer tile, U of
+// 96 MB and more): the input transform in front of it stores V with nt.
+bool wgemm_streams_u(int K, int Cp, int BP);
 // Kernel name (template configuration) launch_wgemm picks for this shape.
 const char* wgemm_name(int K, int Cp, int BP);
 // GEMV-like shapes (BP <= 32, or 48 above K = 1024; U block copy under

@@ -820,7 +820,7 @@ static bool latency_bound(int64_t rows, int n, int ch) { return widest_grid(rows
 
 hipError_t launch_input_transform(const uint16_t* x, uint16_t* V, int B, int C, int H, int W,
                                   int pad, int nh, int nw, int ldv, int64_t pstride,
-                                  hipStream_t s, bool nhwc, bool stream_v, int vfrag) {
+                                  hipStream_t s, bool nhwc, int stream_v, int vfrag) {
     // The two-pass block layout from the run form when its grid fills the
     // CUs (whole forwards in a graph, us, tile-block vs run form: conv3_x
     // batch 32 24.25 vs 23.41 (input transform 8.78 vs 7.77), batch 24 22.75
@@ -852,7 +852,11 @@ hipError_t launch_input_transform(const uint16_t* x, uint16_t* V, int B, int C, 
     // 23.24; batch 128 256@14^2 49.4 -> 45.8; SD-1.5 320@64^2 batch 2 28.3 ->
     // 25.7, 640->320@64^2 34.2 -> 31.7; SDXL 320@128^2 38.0 -> 35.3.
     const bool whole_lines = vfrag == 0 && tw <= 4 && ldv % 64 == 0;
-    const int pol = whole_lines ? kWT : stream_v ? kNt : 0;
+    // In front of a GEMM that streams a U of 96 MB and more (stream_v 2) nt
+    // wins over writing through: 1280 -> 640@32^2 batch 2 45.8 -> 41.1,
+    // 1920 -> 640@32^2 59.5 -> 56.1 (with a U of 52 MB it loses: 640@64^2 batch
+    // 1 28.7 -> 29.0; 512@28^2 batch 4 21.9 -> 24.7).
+    const int pol = whole_lines && stream_v < 2 ? kWT : stream_v ? kNt : 0;
     auto by_policy = [&](auto tw_c, auto go) {
         constexpr int T = decltype(tw_c)::value;
         if (pol == kWT)

@@ -622,6 +622,10 @@ int wgemm_v_reads(int K, int Cp, int BP) {
     return (K + t - 1) / t;
 }
 
+bool wgemm_streams_u(int K, int Cp, int BP) {
+    return wgemm_cfg(K, Cp, BP) == 9 && 2 * (int64_t)64 * K * Cp >= ((int64_t)96 << 20);
+}
+
 const char* wgemm_name(int K, int Cp, int BP) {
     static const char* names[] = {"wgemm_kernel<2, 1, 2, 1, 4>", "wgemm_lds_kernel<64, 64, 2, 2, 2>",
                                   "wgemm_lds_kernel<128, 128, 2, 4, 2>",
