@@ -290,6 +290,9 @@ __global__ __launch_bounds__(kThreads) void wgrad_direct_kernel(WdArgs a) {
                 f.d[r] = *reinterpret_cast<const u4*>(buf + eo + 16 * (2 - r) * a.Ws);
             if constexpr (kStage == kDirectTail) {
                 const int col = col0 + 8 * seg;
+                // the halves left of the first empty segment of a last strip
+                // are the tail of the row's last chunk
+                if (PAD > 0) f.w[0] = col - 2 < a.W ? f.w[0] : 0u;
 #pragma unroll
                 for (int i = 1; i < 6; i++) f.w[i] = col + 2 * (i - 1) < a.W ? f.w[i] : 0u;
 #pragma unroll

@@ -109,6 +109,37 @@ def test_infinities_stay_in_their_channels(W):
     assert not torch.isfinite(got[3, :, 0, 0]).any()
 
 
+# one strip with and without a masked tail; two strips of 16 segments for 19
+# (the first empty one lies right behind the masked chunk) and for 29; odd
+@pytest.mark.parametrize("W", [24, 38, 150, 226, 151])
+@pytest.mark.parametrize("pad", [0, 1, 2])
+def test_infinities_beside_a_row_stay_in_their_channels(W, pad):
+    """The chunks at a row's end reach into what follows in memory: the first
+    pixels of the next row, and behind a channel's last row those of the next
+    channel. Infinities there reach no other channel's gradient."""
+    print(f"[wgrad direct, infinities] W={W} pad={pad}", flush=True)
+    B, C, K, H = 1, 16, 32, 6
+    Ho, Wo = H + 2 * pad - 2, W + 2 * pad - 2
+    g = torch.Generator().manual_seed(W + pad)
+    x = torch.randn(B, C, H, W, generator=g).half().to(DEV)
+    dy = torch.randn(B, K, Ho, Wo, generator=g).half().to(DEV)
+    base = weight_grad(x, dy, pad, C, K)
+    for row, col in ((0, slice(0, 8)), (H - 1, slice(W - 8, W))):
+        x2 = x.clone()
+        x2[0, 8, row, col] = float("inf")
+        got = weight_grad(x2, dy, pad, C, K)
+        keep = torch.arange(C, device=DEV) != 8
+        assert torch.equal(got[:, keep], base[:, keep])
+        assert not torch.isfinite(got[:, 8]).all()
+    for row, col in ((0, slice(0, 8)), (Ho - 1, slice(Wo - 8, Wo))):
+        dy2 = dy.clone()
+        dy2[0, 8, row, col] = float("-inf")
+        got = weight_grad(x, dy2, pad, C, K)
+        keep = torch.arange(K, device=DEV) != 8
+        assert torch.equal(got[keep], base[keep])
+        assert not torch.isfinite(got[8]).all()
+
+
 @pytest.mark.parametrize("B,C,K,H,W,pad,f32", [
     (3, 33, 31, 7, 7, 1, False), (2, 70, 65, 28, 28, 1, False), (4, 16, 40, 56, 56, 0, False),
     (2, 3, 70, 9, 12, 2, False), (1, 320, 64, 16, 16, 1, False), (2, 8, 9, 10, 10, 1, True),
