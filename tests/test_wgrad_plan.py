@@ -1,0 +1,84 @@
+"""Host rules of the direct weight gradient (wgrad_direct.hip), on the CPU: a
+small program linked with the library's own objects prints the plan of each
+shape.
+
+Lanes with nothing to load use byte offset 2^31, which has to lie past the end
+of every buffer resource. The resource over dY starts (2 - pad) rows of dY
+above the tensor, the one over x up to one 16-byte chunk, and each is as much
+longer.
+"""
+
+import os
+import subprocess
+
+import pytest
+
+PKG = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "nova-wino-amd_amd")
+HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+
+PROGRAM = """
+#include <cstdio>
+#include "nova_internal.h"
+int main() {
+    int B, C, K, H, W, pad;
+    while (std::scanf("%d %d %d %d %d %d", &B, &C, &K, &H, &W, &pad) == 6) {
+        const nova::WgradDirectPlan p = nova::wgrad_direct_plan(B, C, K, H, W, pad, 256);
+        std::printf("%d %d\\n", (int)p.ok, p.lo);
+    }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def plans(tmp_path_factory):
+    d = tmp_path_factory.mktemp("wgrad_plan")
+    src, obj, exe = d / "plan.hip", d / "plan.o", d / "plan"
+    src.write_text(PROGRAM)
+    if not os.path.exists(os.path.join(PKG, "_build", "wgrad_direct.o")):
+        subprocess.run(["make", "-C", PKG], check=True)
+    objs = [os.path.join(PKG, "_build", f) for f in sorted(os.listdir(os.path.join(PKG, "_build")))
+            if f.endswith(".o")]
+    subprocess.run([HIPCC, "-std=c++17", "--offload-host-only", "-I", os.path.join(PKG, "csrc"),
+                    "-c", "-o", str(obj), str(src)], check=True)
+    subprocess.run([HIPCC, "-o", str(exe), str(obj), *objs, "-Wl,-rpath,/opt/rocm/lib"],
+                   check=True)
+
+    def run(shapes):
+        text = "\n".join(" ".join(str(v) for v in s) for s in shapes)
+        out = subprocess.run([str(exe)], input=text, capture_output=True, text=True, check=True)
+        return [tuple(int(v) for v in line.split()) for line in out.stdout.split("\n") if line]
+
+    return run
+
+
+def resource_ends(shape, lo):
+    """Bytes of the two resources, for the first channels (the longest), at an
+    address 2 past a dword."""
+    B, C, K, H, W, pad = shape
+    Ho, Wo = H + 2 * pad - 2, W + 2 * pad - 2
+    x = 2 * B * C * H * W + 16 * lo + 2
+    dy = 2 * B * K * Ho * Wo + 2 * (2 - pad) * Wo + 2
+    return (x + 3) & ~3, (dy + 3) & ~3
+
+
+def test_resources_end_below_the_offset_of_empty_lanes(plans):
+    shapes = [(1, 1, 2, 17897, 30002, 0), (1, 1, 1, 17895, 60000, 1)]
+    # tensors around 2 GiB, by columns, rows, channels and images
+    for pad in (0, 1, 2):
+        for Wo in (40, 1000, 16390, 30000, 60000, 120000):
+            for K, B in ((1, 1), (3, 1), (1, 2)):
+                for d in range(-3, 3):
+                    Ho = (2**31 // (2 * Wo * K * B)) + d
+                    shapes.append((B, 1, K, Ho + 2 - 2 * pad, Wo + 2 - 2 * pad, pad))
+    got = plans(shapes)
+    assert len(got) == len(shapes)
+    for shape, (ok, lo) in zip(shapes, got):
+        if ok:
+            assert max(resource_ends(shape, lo)) <= 2**31, shape
+
+
+def test_smaller_tensors_keep_the_direct_products(plans):
+    shapes = [(32, 64, 64, 56, 56, 1), (1, 1, 1, 17000, 60000, 1), (1, 1, 2, 17000, 30002, 0),
+              (1, 1, 1, 3, 3, 0), (2, 65, 40, 9, 11, 2)]
+    assert [ok for ok, _ in plans(shapes)] == [1] * len(shapes)
+    assert [ok for ok, _ in plans([(1, 4, 4, 8, 8, 3), (0, 4, 4, 8, 8, 1)])] == [0, 0]
