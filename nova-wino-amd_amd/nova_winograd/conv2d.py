@@ -521,8 +521,9 @@ class NovaWinogradConv2d(nn.Module):
             hd.set_weights(weight)
             hd.key = (weakref.ref(weight), key)
             self._weight_version = weight._version
-            # the workspace follows the layer's shape and device: new values of
-            # the same parameter (an optimizer step) keep it
+            # the workspace follows the layer's shape and device (and
+            # _ensure_workspace's stream): new values of the same parameter (an
+            # optimizer step) keep it
             if ref is None or ref[1][3:] != key[3:]:
                 self._V_gemm = None
                 self._M_gemm = None
@@ -531,9 +532,18 @@ class NovaWinogradConv2d(nn.Module):
     def _ensure_workspace(self, batch, H, W):
         """Allocate the reference-sized workspace when the configuration
         changes (/root/reference/nova_winograd/conv2d.py:205-220). Layers
-        served by the fused kernel need none."""
-        config = (batch, H, W, self.padding)
-        if self._last_config != config:
+        served by the fused kernel need none.
+
+        The workspace is used on the stream it was allocated on and on no
+        other, so the caching allocator may hand it on in that stream's order
+        when it is dropped. A call in a graph capture takes its own from the
+        graph's pool, and the next call outside takes another: replays write
+        to memory that no later call of the module gives up."""
+        capturing = torch.cuda.is_current_stream_capturing()
+        config = (batch, H, W, self.padding, self._handle.stream)
+        if capturing or self._last_config != config:
+            self._last_config = self._state = None
+            self._V_gemm = self._M_gemm = None
             nh, nw, H_out, W_out = compute_tiling(H, W, self.padding)
             BP = batch * nh * nw
             lib = self._handle.lib
@@ -545,10 +555,9 @@ class NovaWinogradConv2d(nn.Module):
                                            device=device)
                 self._M_gemm = torch.empty(64, self.out_channels, BP, dtype=torch.float16,
                                            device=device)
-            else:
-                self._V_gemm = self._M_gemm = None
             self._tiling = (nh, nw, H_out, W_out)
-            self._last_config = config
+            if not capturing:
+                self._last_config = config
         return self._tiling
 
     # -- forward ------------------------------------------------------------
@@ -618,17 +627,22 @@ class NovaWinogradConv2d(nn.Module):
             "Input must be contiguous (NCHW) or channels_last"
         assert x.dim() == 4 and x.shape[1] == self.in_channels
         out = self._run(x, self.bias, residual)
-        if residual is None and x.is_contiguous():
+        if residual is None and x.is_contiguous() and self._last_config is not None:
             self._remember(x)
         else:
-            # the next call resets the residual / layout on the full path
+            # the next call resets the residual / layout on the full path, or
+            # takes a workspace of its own after one of a graph capture
             self._state = None
         return out
 
     def _remember(self, x):
         """Record what the fast path of ``forward`` checks and replays. The
         weight and bias objects are held, so their identities cannot be
-        reused by other tensors while the record exists."""
+        reused by other tensors while the record exists. The fast path does
+        not look for a capture (0.3 us a call): a graph captured on the very
+        stream of the last eager call replays on that call's workspace, and
+        one captured on a stream of its own, as ``torch.cuda.graph`` does by
+        itself, on its own."""
         hd = self._handle
         B, C, H, W = x.shape
         nh, nw, H_out, W_out = self._tiling
