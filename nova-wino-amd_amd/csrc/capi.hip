@@ -1097,8 +1097,8 @@ void weight_grad_impl(nova_handle_t h, const void* d_input, const void* d_grad_o
     // launch of their own
     if (d_grad_bias != nullptr && !(dp.ok && dp.bias) &&
         !hip_ok(launch_bias_grad(d_grad_output, grad_f32 != 0, static_cast<float*>(d_grad_bias),
-                                 batch, K, (int64_t)(H + 2 * pad - 2) * (W + 2 * pad - 2),
-                                 Hd->stream),
+                                 batch, C, K, (int64_t)(H + 2 * pad - 2) * (W + 2 * pad - 2),
+                                 static_cast<float*>(d_grad_weight), cus, Hd->stream),
                 "bias gradient"))
         return;
     if (dp.ok) {

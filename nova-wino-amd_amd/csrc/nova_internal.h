@@ -325,8 +325,10 @@ WgradDirectPlan wgrad_direct_plan(int B, int C, int K, int H, int W, int pad, in
 hipError_t launch_wgrad_direct(const uint16_t* x, const uint16_t* dy, float* dw, float* db, int B,
                                int C, int K, int H, int W, int pad, const WgradDirectPlan& plan,
                                void* ws, hipStream_t s);
-// db[k] = sum of dY over images and pixels (fp16, or fp32 if dy_f32), fp32.
-hipError_t launch_bias_grad(const void* dy, bool dy_f32, float* db, int B, int K, int64_t HoWo,
-                            hipStream_t s);
+// db[k] = sum of dY over images and pixels (fp16, or fp32 if dy_f32), in fp64.
+// dw: the filter gradient's 9 * K * C floats, to be written later on s; partial
+// sums pass through them, so the sums need no memory of their own.
+hipError_t launch_bias_grad(const void* dy, bool dy_f32, float* db, int B, int C, int K,
+                            int64_t HoWo, float* dw, int cus, hipStream_t s);
 
 }  // namespace nova

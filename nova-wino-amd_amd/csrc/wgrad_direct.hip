@@ -484,25 +484,78 @@ __global__ __launch_bounds__(kRedThreads) void wgrad_direct_reduce_kernel(
     (filter ? dw[i] : db[i - n]) = v;
 }
 
-// db[k] = sum of dY[b][k][:] over images and pixels, in fp64, rounded once:
-// one workgroup per channel.
+// db[k] = sum of dY[b][k][:] over images and pixels, in fp64, rounded once.
+// A channel's pixels are `items` runs of at most kBiasRun of one image, each
+// summed by one wave: single elements up to the first 16-byte boundary and
+// behind the last, 16-byte loads between, four in flight. nsplit workgroups
+// share a channel, each a contiguous range of its runs; their partial sums
+// are added by bias_join_kernel (part null: one workgroup, into db).
+// Bound by reading dY once. Measured on MI355X beside nova_weight_grad (us, one
+// workgroup per channel with 2-byte loads -> this, torch's conversion and sum):
+// fp16 32 channels of 64 x 114^2 855 -> 13, 251; 3 of 16 x 514^2 6050 -> 27, 38;
+// 320 of 8 x 66^2 42 -> 5, 28; 512 of 32 x 9^2 7 -> 8, 14; fp32 32 of 64 x 112^2
+// 1270 -> 25, 219.
+constexpr int kBiasThreads = 512, kBiasRun = 8192;
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) v += __shfl_down(v, d, 64);
+    return v;
+}
 template <typename T>
-__global__ __launch_bounds__(256) void bias_grad_kernel(const T* __restrict__ dy,
-                                                        float* __restrict__ db, int B, int K,
-                                                        int64_t HoWo) {
-    __shared__ double s[256];
-    const int k = (int)blockIdx.x, tid = threadIdx.x;
+__global__ __launch_bounds__(kBiasThreads) void bias_grad_kernel(
+    const T* __restrict__ dy, float* __restrict__ db, double* __restrict__ part, int K,
+    int64_t HoWo, int runs, int64_t items, int nsplit) {
+    constexpr int kE = 16 / sizeof(T), kWaves = kBiasThreads / 64;
+    typedef T vec __attribute__((ext_vector_type(kE)));
+    __shared__ double s[kWaves];
+    const int k = (int)blockIdx.x / nsplit, sp = (int)blockIdx.x - k * nsplit;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t j = (int64_t)sp * kWaves + wave, nj = (int64_t)nsplit * kWaves;
     double v = 0.0;
-    for (int b = 0; b < B; b++) {
-        const T* p = dy + ((int64_t)b * K + k) * HoWo;
-        for (int64_t i = tid; i < HoWo; i += 256) v += (double)p[i];
+    for (int64_t it = j * items / nj; it < (j + 1) * items / nj; it++) {
+        const int64_t b = it / runs, at = (it - b * runs) * kBiasRun;
+        const int n = (int)min((int64_t)kBiasRun, HoWo - at);
+        const T* const p = dy + (b * K + k) * HoWo + at;
+        const int to16 = (int)((0 - reinterpret_cast<uintptr_t>(p)) & 15) / (int)sizeof(T);
+        const int head = min(to16, n), nv = (n - head) / kE, tail = n - head - nv * kE;
+        const vec* const q = reinterpret_cast<const vec*>(p + head);
+        if (lane < head) v += (double)p[lane];
+        if (lane < tail) v += (double)p[n - tail + lane];
+        for (int i = lane; i < nv; i += 256) {
+            vec r[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) r[u] = q[min(i + 64 * u, nv - 1)];
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (i + 64 * u < nv)
+#pragma unroll
+                    for (int e = 0; e < kE; e++) v += (double)r[u][e];
+        }
     }
-    s[tid] = v;
-    for (int d = 128; d > 0; d >>= 1) {
-        __syncthreads();
-        if (tid < d) s[tid] += s[tid + d];
+    v = wave_sum(v);
+    if (lane == 0) s[wave] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        v = s[0];
+        for (int w = 1; w < kWaves; w++) v += s[w];
+        if (part != nullptr)
+            part[blockIdx.x] = v;
+        else
+            db[k] = (float)v;
     }
-    if (tid == 0) db[k] = (float)s[0];
+}
+
+// db[k] = sum of a channel's nsplit partial sums; one wave per channel.
+__global__ __launch_bounds__(256) void bias_join_kernel(const double* __restrict__ part,
+                                                        float* __restrict__ db, int K,
+                                                        int nsplit) {
+    const int k = (int)blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (k >= K) return;
+    double v = 0.0;
+    for (int i = lane; i < nsplit; i += 64) v += part[(int64_t)k * nsplit + i];
+    v = wave_sum(v);
+    if (lane == 0) db[k] = (float)v;
 }
 
 inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
@@ -641,15 +694,35 @@ static hipError_t launch_pad(const WdArgs& a, const WgradDirectPlan& p, int stag
     return launch_direct<PAD, 2, 2>(a, stage, s);
 }
 
-hipError_t launch_bias_grad(const void* dy, bool dy_f32, float* db, int B, int K, int64_t HoWo,
-                            hipStream_t s) {
-    if (dy_f32)
-        launch(bias_grad_kernel<float>, dim3((unsigned)K), dim3(256), s,
-               static_cast<const float*>(dy), db, B, K, HoWo);
-    else
-        launch(bias_grad_kernel<_Float16>, dim3((unsigned)K), dim3(256), s,
-               static_cast<const _Float16*>(dy), db, B, K, HoWo);
+template <typename T>
+static hipError_t launch_bias(const void* dy, float* db, int B, int C, int K, int64_t HoWo,
+                              float* dw, int cus, hipStream_t s) {
+    // Splits: four workgroups per CU in all, at least one run per wave, and as
+    // many fp64 partial sums as dw holds; channels of up to 16384 values are
+    // one workgroup's, without the second launch.
+    const int64_t runs = (HoWo + kBiasRun - 1) / kBiasRun, items = B * runs;
+    int64_t ns = 1;
+    if (B * HoWo > 2 * kBiasRun) {
+        constexpr int kWaves = kBiasThreads / 64;
+        ns = std::min<int64_t>((4 * (int64_t)cus + K - 1) / K, (items + kWaves - 1) / kWaves);
+        ns = std::max<int64_t>(1, std::min<int64_t>(ns, (9 * (int64_t)C - 1) / 2));
+    }
+    double* const part =
+        ns > 1 ? reinterpret_cast<double*>((reinterpret_cast<uintptr_t>(dw) + 7) & ~(uintptr_t)7)
+               : nullptr;
+    launch(bias_grad_kernel<T>, dim3((unsigned)(K * ns)), dim3(kBiasThreads), s,
+           static_cast<const T*>(dy), db, part, K, HoWo, (int)runs, items, (int)ns);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || ns == 1) return e;
+    launch(bias_join_kernel, dim3((unsigned)((K + 3) / 4)), dim3(256), s,
+           static_cast<const double*>(part), db, K, (int)ns);
     return hipGetLastError();
+}
+
+hipError_t launch_bias_grad(const void* dy, bool dy_f32, float* db, int B, int C, int K,
+                            int64_t HoWo, float* dw, int cus, hipStream_t s) {
+    return dy_f32 ? launch_bias<float>(dy, db, B, C, K, HoWo, dw, cus, s)
+                  : launch_bias<_Float16>(dy, db, B, C, K, HoWo, dw, cus, s);
 }
 
 hipError_t launch_wgrad_direct(const uint16_t* x, const uint16_t* dy, float* dw, float* db, int B,

@@ -176,3 +176,93 @@ def test_bias_gradient(B, C, K, H, W, pad, f32):
     want = dy.double().sum(dim=(0, 2, 3))
     bound = (B * Ho * Wo / 8 + 264) * 2.0**-24 * dy.double().abs().sum(dim=(0, 2, 3))
     assert ((gb.double() - want).abs() <= bound).all()
+
+
+def bias_grads(x, dy, pad, K, C, runs=0):
+    """nova_weight_bias_grad's results; with `runs`, also the time it takes
+    beyond nova_weight_grad and torch's own sums, in us."""
+    from nova_winograd.ops import check, get_lib
+
+    lib = get_lib()
+    B, _, H, W = x.shape
+    gw = torch.full((K, C, 3, 3), float("nan"), device=DEV)
+    gb = torch.full((K,), float("nan"), device=DEV)
+    args = (B, C, K, H, W, pad, 1 if dy.dtype == torch.float32 else 0)
+    h = lib.nova_create()
+
+    def us(call):
+        call()
+        best = float("inf")
+        for _ in range(3):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(runs):
+                call()
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b) * 1e3 / runs)
+        return best
+
+    def alone():
+        lib.nova_weight_grad(h, x.data_ptr(), dy.data_ptr(), gw.data_ptr(), *args)
+
+    def both():
+        lib.nova_weight_bias_grad(h, x.data_ptr(), dy.data_ptr(), gw.data_ptr(), gb.data_ptr(),
+                                  *args)
+
+    try:
+        lib.nova_set_stream(h, torch.cuda.current_stream().cuda_stream)
+        times = None
+        if runs:
+            times = (us(both) - us(alone), us(lambda: dy.float().sum(dim=(0, 2, 3))))
+        alone()
+        want = gw.clone()
+        both()
+        check()
+        torch.cuda.synchronize()
+    finally:
+        lib.nova_destroy(h)
+    assert torch.equal(gw.view(torch.int32), want.view(torch.int32))
+    return gb, times
+
+
+# images of one run and of several, of a whole number of 16-byte words and not,
+# channels of one workgroup and of many; few input channels bound the splits
+@pytest.mark.parametrize("B,C,K,Ho,Wo", [
+    (1, 1, 1, 3, 4), (3, 2, 5, 3, 3), (2, 1, 1, 200, 200), (3, 1, 2, 131, 127), (1, 4, 3, 128, 128),
+    (40, 3, 7, 30, 31), (64, 8, 40, 17, 16), (2, 9, 600, 92, 91), (5, 2, 33, 64, 129)])
+@pytest.mark.parametrize("f32", [False, True])
+def test_bias_sums_of_their_own(B, C, K, Ho, Wo, f32):
+    """The sums that the direct products do not take along (padding 2, float32
+    dY): added in fp64 and rounded once, from any address, whatever stands
+    beside them."""
+    print(f"[bias sums] B={B} C={C} K={K} {Ho}x{Wo} f32={f32}", flush=True)
+    pad = 1 if f32 else 2
+    g = torch.Generator().manual_seed(Ho * Wo + K)
+    H, W = Ho + 2 - 2 * pad, Wo + 2 - 2 * pad
+    x = torch.randn(B, C, H, W, generator=g).half().to(DEV)
+    dy = torch.randn(B, K, Ho, Wo, generator=g).to(DEV)
+    dy = dy if f32 else dy.half()
+    want = dy.double().sum(dim=(0, 2, 3))
+    mag = dy.double().abs().sum(dim=(0, 2, 3))
+    for off in (0, 1, 5):
+        gb, _ = bias_grads(x, offset_copy(dy, off), pad, K, C)
+        bound = 2.0**-24 * want.abs() + B * Ho * Wo * 2.0**-53 * mag
+        assert ((gb.double() - want).abs() <= bound).all()
+    dy[0, 0, 0, 0] = float("inf")
+    gb, _ = bias_grads(x, dy, pad, K, C)
+    assert torch.isinf(gb[0]) and torch.isfinite(gb[1:]).all()
+
+
+@pytest.mark.parametrize("B,C,K,H,pad,f32", [(64, 32, 32, 112, 2, False), (16, 64, 3, 512, 2, False),
+                                             (64, 32, 32, 112, 1, True)])
+def test_bias_sums_fill_the_chip(B, C, K, H, pad, f32):
+    """Few channels of many pixels take no longer than torch's conversion and
+    sum (one workgroup per channel took 3 to 150 times as long)."""
+    Ho = H + 2 * pad - 2
+    x = torch.randn(B, C, H, H, device=DEV).half()
+    dy = torch.randn(B, K, Ho, Ho, device=DEV)
+    dy = dy if f32 else dy.half()
+    _, (own, torchs) = bias_grads(x, dy, pad, K, C, runs=10)
+    print(f"[bias sums] B={B} K={K} {Ho}^2 f32={f32}: {own:.1f} us, torch {torchs:.1f}", flush=True)
+    assert own <= 1.5 * torchs + 20
