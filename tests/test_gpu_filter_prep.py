@@ -3,7 +3,7 @@ oracle's transform, the flipped form against the flipped weights, and both
 fragment-ordered copies against U, at both lane widths (8 channels per lane
 from 512 pairs per CU on, else 2) and at channel counts off the 8, 16, 32 and
 64 blocks. The forwards of the paths that read each copy must agree bit for
-bit with the three-pass path, which reads U."""
+bit with the same paths on copies built from U."""
 
 import numpy as np
 import pytest
@@ -65,11 +65,16 @@ def test_u_and_flipped_u(oracle, K, C, f16):
             lib.nova_destroy(x)
 
 
-@pytest.mark.parametrize("K,C", [(64, 64), (40, 48), (17, 9), (128, 128), (256, 128), (96, 24),
-                                 (512, 512)])
-def test_copies_match_u(K, C):
-    """Paths that read Uf (5, 3) or Uw (6, 7) against path 1, with weights set
-    twice: the second time a handle's copies are written by set_weights."""
+# paths: those that serve 2 x 13^2 with these channels when asked to
+@pytest.mark.parametrize("K,C,paths", [
+    (64, 64, (3, 5, 6, 7)), (40, 48, (3, 5, 6, 7)), (17, 9, (3, 5, 6, 7)), (128, 128, (6, 7)),
+    (256, 128, (6, 7)), (96, 24, (6, 7)), (512, 512, (6, 7))])
+def test_copies_match_u(K, C, paths):
+    """The copies that set_weights writes, Uf (paths 3 and 5) and Uw (6 and 7),
+    against copies built afterwards from U: forwards of the same path, bit for
+    bit. Weights are set twice, since some copies are written by set_weights
+    only once a forward has used them. Paths 6 and 7 also match path 1, which
+    reads U, and 3 and 5 sum the channels in another order."""
     from nova_winograd.ops import check, get_lib
 
     lib = get_lib()
@@ -77,8 +82,19 @@ def test_copies_match_u(K, C):
     B, H = 2, 13
     x = torch.randn(B, C, H, H, generator=g).half().to(DEV)
     w = torch.randn(K, C, 3, 3, generator=g).to(DEV) * 0.05
-    outs = {}
-    for path in (1, 3, 5, 6, 7):
+
+    def forward(h, path):
+        y = torch.empty(B, K, H, H, dtype=torch.float16, device=DEV)
+        lib.nova_forward(h, x.data_ptr(), y.data_ptr(), B, H, H, 1)
+        check()
+        torch.cuda.synchronize()
+        ran = lib.nova_get_last_path(h)
+        print(f"[filter copies] K={K} C={C} asked {path} ran {ran}", flush=True)
+        assert ran == path
+        return y
+
+    def written(path):
+        """set_weights under the path, twice."""
         h = lib.nova_create()
         try:
             lib.nova_set_path(h, path)
@@ -86,19 +102,28 @@ def test_copies_match_u(K, C):
                 ws = w * scale
                 lib.nova_set_weights(h, ws.data_ptr(), K, C)
                 check()
-                y = torch.empty(B, K, H, H, dtype=torch.float16, device=DEV)
-                lib.nova_forward(h, x.data_ptr(), y.data_ptr(), B, H, H, 1)
-                lib.nova_get_last_error()
-                torch.cuda.synchronize()
-            outs[path] = (lib.nova_get_last_path(h), y)
+                y = forward(h, path)
+            return y
         finally:
             lib.nova_destroy(h)
-    for path, (ran, y) in outs.items():
-        print(f"[filter copies] K={K} C={C} asked {path} ran {ran}", flush=True)
-        if ran in (6, 7):
-            assert torch.equal(y, outs[1][1])
-        elif ran in (3, 5):  # another order of the channel sums
-            d = (y.float() - outs[1][1].float()).norm() / outs[1][1].float().norm()
-            assert d <= 5e-3
-    if outs[3][0] == 3 and outs[5][0] == 5:
-        assert torch.equal(outs[3][1], outs[5][1])
+
+    def built(path):
+        """U alone by set_weights, the copy from it when the path is asked for."""
+        h = lib.nova_create()
+        try:
+            lib.nova_set_path(h, 1)
+            lib.nova_set_weights(h, w.data_ptr(), K, C)
+            lib.nova_set_path(h, path)
+            check()
+            return forward(h, path)
+        finally:
+            lib.nova_destroy(h)
+
+    base = built(1)
+    for path in paths:
+        y = written(path)
+        assert torch.equal(y, built(path)), path
+        if path in (6, 7):
+            assert torch.equal(y, base)
+        else:
+            assert (y.float() - base.float()).norm() <= 5e-3 * base.float().norm()
