@@ -151,8 +151,9 @@ constexpr int64_t kWTSmallBytes = (int64_t)2 << 20;
 // V store cache policy (results unchanged): the forms whose wave stores are
 // whole 128-byte lines (the tile-block forms in the product layout with at
 // least 64 channels per workgroup and ldv % 64 == 0, and the run form) write
-// through the L2; otherwise stream_v 1 asks for the non-temporal (nt) policy
-// (see wgemm_v_reads for when it pays); stream_v 2 asks for it in every form.
+// through the L2; otherwise stream_v 1 asks for the non-temporal (nt) policy,
+// and stream_v 2 asks the tile-block forms for it in any case (wgemm_stream_v).
+// The run form and the lane-parallel form of small grids keep their own.
 // vfrag: 0 = V in the product layout V[p][bp][ldv]; otherwise the number of
 // 32-channel chunks of the two-pass layout (1 KB MFMA B-operand blocks of 16
 // tiles x 32 channels; pstride = ceil(BP / 16) * vfrag * 512 halves).
@@ -174,15 +175,23 @@ hipError_t launch_output_transform(const uint16_t* M, uint16_t* y, int B, int K,
 // [64][BP][K].
 hipError_t launch_wgemm(const uint16_t* U, const uint16_t* V, uint16_t* M, int K, int Cp,
                         int BP, hipStream_t s);
-// Times the GEMM reads each V element (its output-channel tiles). Measured on
-// MI355X (whole forwards): streaming V past the L2 pays when this is at most 4
-// (ResNet-50 at batch 32: 128@28^2 31.7 -> 28.9 us, 256@14^2 31.2 -> 30.3,
-// 512@7^2 29.0 -> 28.4) and costs when V is re-read more often (320@128^2 at
-// batch 1, five reads: 43.1 -> 45.1 us; 640@64^2, ten: 36.7 -> 39.1 us).
-int wgemm_v_reads(int K, int Cp, int BP);
-// A deep layer's GEMM whose U streams past the caches (three-buffer tile, U of
-// 96 MB and more): the input transform in front of it stores V with nt.
-bool wgemm_streams_u(int K, int Cp, int BP);
+// stream_v of the input transform in front of this GEMM. 2 (nt in the
+// tile-block forms, whole lines too) where U streams past the caches (the
+// three-buffer tile, U of 96 MB and more). 1 (nt where a wave's stores are
+// pieces of lines: Cp % 64 != 0, or blocks of 8 tiles) for V of up to 24 MB
+// (a larger one is read faster from the L2: batch 128 128@28^2, 52 MB, 61.3
+// against 58.1 us, 512@7^2, 34 MB, 54.7 against 50.9) that the GEMM reads at
+// most 4 times (its rows of tiles), and
+//  * of up to 256 output channels (512 from 256 tiles on);
+//  * above, where the 96- and 160-row tiles read V that rarely: rows of V on
+//    64-byte boundaries (Cp % 32 == 0) and V of at least 12 MB or M of at
+//    least 32 MB. Over 204 such layers nt took 1.02 times as long as plain
+//    stores on average, 1.05 with rows off 64 bytes (328 -> 320@128^2 1.25, 200
+//    -> 480@14^2 batch 48 1.10), and with this rule the mean is 0.998. Whole
+//    forwards in a graph, us, plain against nt: 320@128^2 38.1, 36.5; 96 ->
+//    480@14^2 batch 96 8 % in favour of nt; 160 -> 320@23^2 batch 36 30.1,
+//    31.1.
+int wgemm_stream_v(int K, int Cp, int BP);
 // Kernel name (template configuration) launch_wgemm picks for this shape.
 const char* wgemm_name(int K, int Cp, int BP);
 // GEMV-like shapes (BP <= 32, or 48 above K = 1024; U block copy under

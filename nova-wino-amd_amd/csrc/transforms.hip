@@ -846,8 +846,8 @@ hipError_t launch_input_transform(const uint16_t* x, uint16_t* V, int B, int C, 
     // V stores: a wave writes 64 consecutive channels of one (tile,
     // position) -- whole 128-byte lines in the product layout when the
     // workgroup holds at least 64 channels and rows are whole lines -- written
-    // through the L2 (kWT); otherwise nt when the GEMM reads V few times
-    // (stream_v), else write-back. Whole forwards in a graph, us, before ->
+    // through the L2 (kWT); otherwise nt where the GEMM's rule says so
+    // (stream_v, wgemm_stream_v), else write-back. Whole forwards in a graph, us, before ->
     // after: ResNet-50 batch 32 256@14^2 25.75 -> 24.49, 512@7^2 25.42 ->
     // 23.24; batch 128 256@14^2 49.4 -> 45.8; SD-1.5 320@64^2 batch 2 28.3 ->
     // 25.7, 640->320@64^2 34.2 -> 31.7; SDXL 320@128^2 38.0 -> 35.3.

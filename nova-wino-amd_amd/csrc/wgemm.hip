@@ -616,14 +616,14 @@ static int wgemm_cfg(int K, int Cp, int BP) {
     return K > 256 || (BP >= 128 && Cp >= 256) ? 1 : 4;
 }
 
-int wgemm_v_reads(int K, int Cp, int BP) {
+int wgemm_stream_v(int K, int Cp, int BP) {
     static const int tk[] = {64, 64, 128, 128, 64, 128, 64, 64, 160, 160, 96, 96};
-    const int t = tk[wgemm_cfg(K, Cp, BP)];  // output channels per workgroup tile
-    return (K + t - 1) / t;
-}
-
-bool wgemm_streams_u(int K, int Cp, int BP) {
-    return wgemm_cfg(K, Cp, BP) == 9 && 2 * (int64_t)64 * K * Cp >= ((int64_t)96 << 20);
+    const int cfg = wgemm_cfg(K, Cp, BP);
+    const int64_t v_bytes = 2 * (int64_t)64 * Cp * BP, m_bytes = 2 * (int64_t)64 * K * BP;
+    if (cfg == 9 && 2 * (int64_t)64 * K * Cp >= ((int64_t)96 << 20)) return 2;
+    if (v_bytes > ((int64_t)24 << 20) || (K + tk[cfg] - 1) / tk[cfg] > 4) return 0;
+    if (K <= 256 || (K == 512 && BP >= 256)) return 1;
+    return Cp % 32 == 0 && (v_bytes >= ((int64_t)12 << 20) || m_bytes >= ((int64_t)32 << 20));
 }
 
 const char* wgemm_name(int K, int Cp, int BP) {
