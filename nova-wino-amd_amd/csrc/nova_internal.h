@@ -176,8 +176,10 @@ hipError_t launch_output_transform(const uint16_t* M, uint16_t* y, int B, int K,
 hipError_t launch_wgemm(const uint16_t* U, const uint16_t* V, uint16_t* M, int K, int Cp,
                         int BP, hipStream_t s);
 // stream_v of the input transform in front of this GEMM. 2 (nt in the
-// tile-block forms, whole lines too) where U streams past the caches (the
-// three-buffer tile, U of 96 MB and more). 1 (nt where a wave's stores are
+// tile-block forms, whole lines too) where U streams past the caches: the
+// three-buffer tile with U of 96 MB and more, the one tile it was measured for
+// over the range (the 128 x 64 tile's few layers of 1280 channels: 1280@48^2
+// batch 1 74.0 -> 70.1 us, 1280@32^2 batch 2 77.7 -> 77.3). 1 (nt where a wave's stores are
 // pieces of lines: Cp % 64 != 0, or blocks of 8 tiles) for V of up to 24 MB
 // (a larger one is read faster from the L2: batch 128 128@28^2, 52 MB, 61.3
 // against 58.1 us, 512@7^2, 34 MB, 54.7 against 50.9) that the GEMM reads at
@@ -318,7 +320,8 @@ hipError_t launch_wgrad(const uint16_t* x, const void* dy, bool dy_f32, float* d
 
 // Direct form for fp16 dY (wgrad_direct.hip): nine taps as fp16 MFMA products
 // over the pixels, the operands read as they are, fp32 sums. ok is false
-// where the form does not apply (pads above 2, no images, images of 1 GiB).
+// where the form does not apply (pads above 2, no images, x or dY of 2 GiB less
+// 64 KB and the two rows that dY's resource starts above it).
 struct WgradDirectPlan {
     int wk, wc;         // waves along output and input channels (of 8)
     int G, R, nrb;      // images and x rows per unit, row blocks per image
