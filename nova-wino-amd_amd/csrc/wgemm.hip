@@ -549,12 +549,13 @@ const char* wgemm_blocks_name(int BP) {
 // every tile shape on MI355X (GEMM launches inside forwards, per-kernel
 // events, us; the results are bit-identical across tile shapes). Tiles that
 // leave no more of K empty than 64-row ones, as large as the work allows:
-//  * 160 x 128 where 160 divides K as well as 64 does, from 240 tiles (128
-//    above K = 1024): fewer and larger workgroups read V and U less often
+//  * 160 x 128 where 160 divides K as well as 64 does, from 240 tiles with a
+//    workgroup for every CU (128 above K = 1024): fewer and larger workgroups read V and U less often
 //    (320@64^2 B=16 60.3 for 64 x 128, 59.5 for 128 x 128, 51.0; B=8 33.4,
 //    31.5, 27.4; 640@64^2 B=8 91.1, 81.8, 73.3; 160@28^2 B=32 13.1, 11.7,
 //    10.4; 1280@32^2 B=4, 144 tiles, 76.5 for 64 x 96, 72.1, 66.6); below
-//    that the grid is too small (640@64^2 B=1, 121 tiles: 14.6 against 13.6);
+//    that the grid is too small (640@64^2 B=1, 121 tiles: 14.6 against 13.6;
+//    64 -> 160@24^2 B=16, 128 workgroups, a forward 17.1 against 16.2);
 //  * the same tile with three buffers for deep layers at 64 to 128 tiles (U
 //    streams from memory, one workgroup per CU: 1280 -> 640@32^2 B=2 27.6
 //    against 30.2 with two buffers and 32.1 for 64 x 96; 640@64^2 B=1 12.3
@@ -565,16 +566,26 @@ const char* wgemm_blocks_name(int BP) {
 //    forwards, eager, us: 384@20^2 B=12 24.9 for 64 x 64, 21.9; 480@30^2 B=6
 //    31.9, 30.0; 192@28^2 B=32 34.4 for 64 x 128, 96 x 128 34.5, 96 x 96 33.5;
 //    launch alone 96@56^2 B=16 12.7 for 64 x 128, 96 x 96 10.7, 96 x 128 9.7;
-//    384@28^2 B=8 9.0, 9.5, 8.2), the width that fills BP better;
+//    384@28^2 B=8 9.0, 9.5, 8.2), the width that fills BP better; up to K =
+//    192 from 384 tiles, below which the grid is too small (whole forwards in a
+//    graph: 480 -> 96@48^2 B=2 21.5 against 18.9 for 64 x 64, 96@14^2 B=16 12.5
+//    and 11.7, 192@40^2 B=3 17.0 and 16.4); from K = 640 and 256 tiles, where
+//    128 x 128 begins, only if 96 tiles fill BP 15 points better (768@56^2 B=4,
+//    400 tiles, 100.3 against 87.7, 640 -> 768@64^2 B=4, 484, 99.8 and 91.2; 64 ->
+//    768@14^2 B=32, 288 tiles, 23.0 and 24.1);
 //  * 128 rows where 128 divides K as well: 128 x 192 from 500 tiles that it
 //    fills (256@14^2 B=64 27.2 -> 26.4, B=128 54.0 -> 51.6 for whole
 //    forwards), 128 x 128 from 300 (48 -> 200@21^2 B=20 19.0 -> 18.1), for
 //    K >= 512 from 256 (512@7^2 B=64 13.9 vs 15.5-17.3 for the other shapes,
 //    B=128 24.9 vs 26.2-30.8), for K of 97 to 128 from 1600 (128@28^2 B=64
 //    10.7 for 64 x 128, 10.2, B=128 25.4, 22.8);
-//  * 128 x 64 (8 waves) for K >= 1024 below 128 tiles (a register-staged
-//    form: 1280@16^2 B=2 33.6 vs 36.4 for 64 x 64; 1280@32^2 B=1 34.0 vs
-//    35.9; 640->1280@16^2 B=2 17.8 vs 19.5);
+//  * 128 x 64 (8 waves) for K >= 1024 below 128 tiles (whole forwards, us,
+//    against 64 x 64, 64 x 128 and 64 x 96: 1280@48^2 B=1 74.0 vs 78.2, 79.4,
+//    78.9; 1280@32^2 B=2 77.7 vs 83.5, 80.9, 79.5; 1024@48^2 B=1 46.5 vs 48.0,
+//    54.7, 49.0; up to 32 tiles, or 48 above K = 1024, the operand-block kernel
+//    takes them). The three-buffer 160 x 128 tile, which stops below K = 1024, is
+//    faster still where 160 divides K (67.8 and 69.1 at the first two) and
+//    slower where it does not (51.0 at the third);
 //  * 64 x 128 for larger work: K >= 640 from 64 tiles, K >= 512 from 128,
 //    K >= 256 from 200 (512@7^2 B=32 9.0 vs 10.0 for 128 x 128; 256@14^2 B=24
 //    18.7 vs 19.0);
@@ -582,24 +593,31 @@ const char* wgemm_blocks_name(int BP) {
 //    points better than 128, for K >= 256 from 128 tiles (256@14^2 B=32, 288
 //    tiles, 6.6 against 7.5, B=16 16.3 -> 15.9 for a forward; 640@32^2 B=2, 72
 //    tiles, 11.4 against 12.4);
-//  * else 64 x 64: four waves above K = 256 or from 128 tiles and four stages
-//    (512@7^2 B=16 7.8 against 8.0), else eight (with one or two stages four
-//    lost 1.5-4 % of a forward: 48 -> 200@21^2 B=20, 128@56^2 B=2). Odd
-//    channel counts (K % 8 != 0, M stored in pieces) stay with 64 rows
-//    (189@15^2 B=45 28.5 against 30.0 for 96 x 128).
+//  * else 64 x 64: four waves from 300 workgroups, eight below (210 layers that
+//    the rules above leave: up to 300 eight take 2 % of a forward less, at 300 to
+//    400 they are equal, above that four take 1-4 % less). Channel
+//    counts off 8 (M stored in pieces) have only the rules without fill: 64
+//    rows (189@15^2 B=45 28.5 against 30.0 for 96 x 128), and the 128-row tiles
+//    of K >= 512 from 256 tiles and K >= 1024 below 128 (517@33^2 B=9 45.9
+//    against 44.2 for 64 rows, 1029@33^2 B=16 119.9 against 119.0-122.6, 1030@25^2
+//    B=2 45.4 against 45.7-48.5).
 // Share of a row of tiles of width t that n fills.
 static double fill(int n, int t) { return (double)n / (t * ((n + t - 1) / t)); }
 
 static int wgemm_cfg(int K, int Cp, int BP) {
     if (BP <= 16) return 0;
     const bool narrow = fill(BP, 96) >= fill(BP, 128) + 0.15;
+    const auto grid = [=](int tk, int tb) {  // workgroups
+        return (int64_t)64 * ((K + tk - 1) / tk) * ((BP + tb - 1) / tb);
+    };
     if (K % 8 == 0) {
         if (K >= 160 && fill(K, 160) >= fill(K, 64)) {
-            if (BP >= 240 || (K >= 1024 && BP >= 128)) return 8;
+            if ((BP >= 240 && grid(160, 128) >= 256) || (K >= 1024 && BP >= 128)) return 8;
             if (K >= 640 && K < 1024 && Cp >= (narrow ? 1024 : 640) && BP >= 64 && BP <= 128)
                 return 9;
         }
-        if (BP >= 128 && K >= 65 && fill(K, 96) >= std::max(fill(K, 64), fill(K, 128)))
+        if (BP >= 128 && K >= 65 && fill(K, 96) >= std::max(fill(K, 64), fill(K, 128)) &&
+            (K > 192 || BP >= 384) && (K < 640 || BP < 256 || narrow))
             return fill(BP, 96) >= fill(BP, 128) + 0.03 ? 11 : 10;
         if (K >= 192 && fill(K, 128) >= fill(K, 64)) {
             if (BP >= 500 && fill(BP, 192) >= fill(BP, 128)) return 3;
@@ -613,7 +631,7 @@ static int wgemm_cfg(int K, int Cp, int BP) {
     if ((K >= 640 && BP >= 64) || (K >= 512 && BP >= 128) || (K >= 256 && BP >= 200) ||
         (K <= 128 && BP >= 1600))
         return narrow ? 7 : 6;
-    return K > 256 || (BP >= 128 && Cp >= 256) ? 1 : 4;
+    return grid(64, 64) >= 300 ? 1 : 4;
 }
 
 int wgemm_stream_v(int K, int Cp, int BP) {

@@ -17,13 +17,13 @@ pytestmark = pytest.mark.gpu
 
 # (B, C, K, H, kernel): BP = B * ceil(H / 6)^2
 CASES = [
-    (3, 40, 168, 54, "<96, 128, 2, 4, 2>"),    # BP 243, K past a tile
+    (9, 40, 280, 28, "<96, 128, 2, 4, 2>"),    # BP 225, K past a tile
     (5, 300, 200, 33, "<64, 64, 2, 2, 2>"),    # BP 180
     (3, 72, 320, 54, "<160, 128, 2, 4, 2>"),   # BP 243, two stages, the last of 8 channels
     (2, 700, 640, 36, "<64, 96, 2, 2, 2>"),    # BP 72, 11 stages
     (2, 1030, 640, 33, "<160, 128, 2, 4, 3>"),  # three buffers; channels end inside a stage
-    (6, 136, 96, 30, "<96, 96, 2, 2, 2>"),     # BP 150
-    (9, 64, 192, 28, "<96, 128, 2, 4, 2>"),    # BP 225, one stage
+    (6, 136, 288, 30, "<96, 96, 2, 2, 2>"),    # BP 150
+    (9, 64, 480, 28, "<96, 128, 2, 4, 2>"),    # BP 225, one stage
     (16, 64, 256, 36, "<128, 192, 2, 4, 2>"),  # BP 576
     (9, 200, 512, 33, "<128, 128, 2, 4, 2>"),  # BP 324
     (2, 129, 1032, 25, "<128, 64, 2, 4, 2>"),  # BP 50, K past a tile
@@ -31,7 +31,7 @@ CASES = [
     (9, 72, 696, 30, "<64, 128, 2, 4, 2>"),    # BP 225, K past a tile
     (1, 24, 40, 36, "<64, 64, 2, 4, 2>"),      # BP 36, M staged
     # K % 8 != 0: M stored in pieces of four channels, or one by one (odd K)
-    (8, 66, 130, 25, "<64, 64, 2, 4, 2>"),     # BP 200
+    (8, 66, 130, 25, "<64, 64, 2, 2, 2>"),     # BP 200
     (5, 9, 33, 30, "<64, 64, 2, 4, 2>"),       # BP 125, one partial stage
     (9, 77, 700, 30, "<64, 128, 2, 4, 2>"),    # BP 225
     (9, 40, 517, 33, "<128, 128, 2, 4, 2>"),   # BP 324

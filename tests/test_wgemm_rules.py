@@ -1,8 +1,7 @@
-"""The cache policy of the V stores in front of the Winograd-domain GEMM
-(wgemm_stream_v), a host rule, on the CPU: 0 plain, 1 nt where stores are
-pieces of lines, 2 nt in any case. Layers of more than 256 channels that the
-96- and 160-row tiles read few times were slower with nt unless V's rows lie on
-64-byte boundaries and V or M is large."""
+"""Host rules of the Winograd-domain GEMM, on the CPU: the tile it takes
+(wgemm_name) and the cache policy of the V stores in front of it
+(wgemm_stream_v: 0 plain, 1 nt where stores are pieces of lines, 2 nt in any
+case). Each case is a layer whose time was measured on both sides."""
 
 import pytest
 
@@ -13,16 +12,50 @@ PROGRAM = """
 #include "nova_internal.h"
 int main() {
     int K, Cp, BP;
-    while (std::scanf("%d %d %d", &K, &Cp, &BP) == 3)
-        std::printf("%d\\n", nova::wgemm_stream_v(K, Cp, BP));
+    while (std::scanf("%d %d %d", &K, &Cp, &BP) == 3) {
+        int tk = 0, tb = 0, wk = 0, wb = 0;
+        std::sscanf(nova::wgemm_name(K, Cp, BP), "wgemm_lds_kernel<%d, %d, %d, %d", &tk, &tb, &wk,
+                    &wb);
+        std::printf("%d %d %d %d\\n", nova::wgemm_stream_v(K, Cp, BP), tk, tb, wk * wb);
+    }
 }
 """
 
 
 @pytest.fixture(scope="module")
-def stream_v(tmp_path_factory):
-    run = build(tmp_path_factory.mktemp("wgemm_rules"), PROGRAM)
-    return lambda rows: [v for v, in run(rows)]
+def rules(tmp_path_factory):
+    return build(tmp_path_factory.mktemp("wgemm_rules"), PROGRAM)
+
+
+@pytest.fixture(scope="module")
+def stream_v(rules):
+    return lambda rows: [r[0] for r in rules(rows)]
+
+
+@pytest.fixture(scope="module")
+def tile(rules):
+    return lambda rows: [r[1:] for r in rules(rows)]
+
+
+def test_96_row_tiles_need_workgroups(tile):
+    # (K, Cp, BP): 96 of 72 or 96 channels left most CUs idle (480 -> 96@48^2
+    # batch 2 18.7 -> 21.4 us); so did 160 rows of 160 channels
+    assert tile([(96, 480, 128), (72, 72, 128), (96, 96, 144), (192, 192, 147),
+                 (160, 64, 256)]) == [(64, 64, 8)] * 2 + [(64, 64, 4)] * 3
+    assert tile([(96, 448, 576), (192, 192, 512), (288, 288, 192), (384, 384, 144),
+                 (160, 160, 800)]) == [(96, 96, 4), (96, 128, 8), (96, 96, 4), (96, 96, 4),
+                                       (160, 128, 8)]
+
+
+def test_wide_layers_take_128_rows_from_256_tiles(tile):
+    # 640 -> 768@64^2 batch 4 94.6 -> 102.1 us with 96 rows, 768@56^2 likewise
+    assert tile([(768, 640, 484), (768, 768, 400), (768, 64, 288), (768, 768, 192)]) == [
+        (128, 128, 8), (128, 128, 8), (96, 96, 4), (96, 96, 4)]
+
+
+def test_64_row_tiles_take_four_waves_from_300_workgroups(tile):
+    assert tile([(128, 128, 128), (200, 200, 144), (333, 336, 64), (576, 576, 50),
+                 (64, 64, 1024)]) == [(64, 64, 8)] + [(64, 64, 4)] * 4
 
 
 def test_wide_layers_off_64_bytes_or_small_are_not_streamed(stream_v):
