@@ -109,6 +109,7 @@ struct Handle {
     uint16_t* Uw = nullptr;  // U in 1 KB operand blocks (two-pass kernel, GEMV-like GEMMs)
     size_t Uw_cap = 0;       // bytes
     bool uw_ready = false;   // Uw holds the current weights' blocks
+    bool uw_used = false;    // a forward has asked for them since set_weights
     void* ws = nullptr;
     size_t ws_cap = 0;  // bytes
     unsigned* cnt = nullptr;  // fused-kernel arrival counters, zero between launches
@@ -220,6 +221,7 @@ bool ensure_uf(Handle* H) {
 // Uf: at set_weights when the automatic choice can pick path 6 or it is
 // forced, else on the first forward that needs it.
 bool ensure_uw(Handle* H) {
+    H->uw_used = true;
     if (H->uw_ready) return true;
     if (!alloc_uw(H)) return false;
     H->uw_ready = hip_ok(launch_u_wfrag(H->U, H->Uw, H->K, H->Cp, H->stream),
@@ -969,9 +971,12 @@ void set_weights_impl(nova_handle_t h, const void* d_weight, int K, int C, bool 
         }
         H->U_cap = need;
     }
-    // new weights of the layer whose last ones got their operand blocks in a
-    // forward (or here) will need them again
-    const bool again = H->uw_ready && H->K == K && H->C == C;
+    // new weights of a layer whose last ones were read as operand blocks will
+    // be again; where they were not (another batch size since), the blocks are
+    // left to a forward that needs them: at 1280 x 1280 writing them takes as
+    // long as the rest of a batch-8 16^2 pass (118 -> 242 us)
+    const bool again = H->uw_used && H->K == K && H->C == C;
+    H->uw_used = false;
     H->uf_ready = false;
     H->uw_ready = false;
     H->K = K;

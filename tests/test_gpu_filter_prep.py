@@ -127,3 +127,43 @@ def test_copies_match_u(K, C, paths):
             assert torch.equal(y, base)
         else:
             assert (y.float() - base.float()).norm() <= 5e-3 * base.float().norm()
+
+
+def test_blocks_are_written_only_while_forwards_read_them():
+    """One batch-1 forward reads U's operand blocks; the steps at a larger
+    batch that follow, each with new weights, take as long as on a handle that
+    never had them (they took twice as long while set_weights went on writing
+    the blocks)."""
+    from nova_winograd.ops import check, get_lib
+
+    lib = get_lib()
+    C, B, H = 1280, 8, 16
+    w = torch.randn(C, C, 3, 3, device=DEV) * 0.02
+    x, one = (torch.randn(n, C, h, h, device=DEV).half() for n, h in ((B, H), (1, 7)))
+    y, y1 = torch.empty_like(x), torch.empty_like(one)
+
+    def step_us(batch_1_first):
+        h = lib.nova_create()
+        try:
+            lib.nova_set_stream(h, torch.cuda.current_stream().cuda_stream)
+            lib.nova_set_weights(h, w.data_ptr(), C, C)
+            if batch_1_first:
+                lib.nova_forward(h, one.data_ptr(), y1.data_ptr(), 1, 7, 7, 1)
+            best = float("inf")
+            for _ in range(4):
+                a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+                a.record()
+                for _ in range(10):
+                    lib.nova_set_weights(h, w.data_ptr(), C, C)
+                    lib.nova_forward(h, x.data_ptr(), y.data_ptr(), B, H, H, 1)
+                b.record()
+                torch.cuda.synchronize()
+                best = min(best, a.elapsed_time(b) * 100)
+            check()
+            return best
+        finally:
+            lib.nova_destroy(h)
+
+    fresh, after = step_us(False), step_us(True)
+    print(f"[filter blocks] fresh {fresh:.1f} us, after a batch-1 forward {after:.1f}", flush=True)
+    assert after <= 1.4 * fresh
