@@ -75,7 +75,8 @@ hipError_t launch_filter_transform_ref(const float* w, uint16_t* U, int K, int C
     return hipGetLastError();
 }
 
-// Filter transform into everything a layer's kernels read, in one launch: the
+// Filter transform into everything a layer's kernels read, in one launch (the
+// largest unflipped layers' in two, launch_filter_prep): the
 // product layout U[p][k][Cp] and, where not null, the two fragment-ordered
 // copies (launch_u_frag's Uf, launch_u_wfrag's Uw) with their zero padding.
 // kFlip: the filter of the input gradient, read from the layer's own weights
@@ -196,6 +197,19 @@ static hipError_t launch_prep(const WT* w, bool flip, uint16_t* U, uint16_t* Uf,
 
 hipError_t launch_filter_prep(const void* w, bool w_f16, bool flip, uint16_t* U, uint16_t* Uf,
                               uint16_t* Uw, int K, int C, int Cp, int cus, hipStream_t s) {
+    // From 96 MB of U on, the copies of unflipped weights by launches of their
+    // own (U and Uw, us, one launch against two: 832 x 832 36 and 45; 640 x 1280
+    // 71 and 61, 896 x 896 70 and 60, 1280 x 1280 180 and 134, 2560 x 1280 356
+    // and 249). Flipped, where U alone comes from this kernel too, one launch
+    // holds to 1024 x 1024 (with a gradient behind it 120 and 131; 1280 x 1280
+    // 222 and 207).
+    if (!flip && (Uf != nullptr || Uw != nullptr) &&
+        2 * (int64_t)64 * K * Cp >= ((int64_t)96 << 20)) {
+        hipError_t e = launch_filter_prep(w, w_f16, flip, U, nullptr, nullptr, K, C, Cp, cus, s);
+        if (e == hipSuccess && Uf != nullptr) e = launch_u_frag(U, Uf, K, Cp, s);
+        if (e == hipSuccess && Uw != nullptr) e = launch_u_wfrag(U, Uw, K, Cp, s);
+        return e;
+    }
     if (!flip && Uf == nullptr && Uw == nullptr) {
         const dim3 grid((unsigned)(((int64_t)K * Cp + 255) / 256));
         if (w_f16)

@@ -68,7 +68,8 @@ def test_u_and_flipped_u(oracle, K, C, f16):
 # paths: those that serve 2 x 13^2 with these channels when asked to
 @pytest.mark.parametrize("K,C,paths", [
     (64, 64, (3, 5, 6, 7)), (40, 48, (3, 5, 6, 7)), (17, 9, (3, 5, 6, 7)), (128, 128, (6, 7)),
-    (256, 128, (6, 7)), (96, 24, (6, 7)), (512, 512, (6, 7))])
+    (256, 128, (6, 7)), (96, 24, (6, 7)), (512, 512, (6, 7)),
+    (1000, 800, (6,))])
 def test_copies_match_u(K, C, paths):
     """The copies that set_weights writes, Uf (paths 3 and 5) and Uw (6 and 7),
     against copies built afterwards from U: forwards of the same path, bit for
