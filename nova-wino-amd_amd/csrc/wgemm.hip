@@ -595,12 +595,14 @@ const char* wgemm_blocks_name(int BP) {
 //    tiles, 11.4 against 12.4);
 //  * else 64 x 64: four waves from 300 workgroups, eight below (210 layers that
 //    the rules above leave: up to 300 eight take 2 % of a forward less, at 300 to
-//    400 they are equal, above that four take 1-4 % less). Channel
-//    counts off 8 (M stored in pieces) have only the rules without fill: 64
-//    rows (189@15^2 B=45 28.5 against 30.0 for 96 x 128), and the 128-row tiles
-//    of K >= 512 from 256 tiles and K >= 1024 below 128 (517@33^2 B=9 45.9
-//    against 44.2 for 64 rows, 1029@33^2 B=16 119.9 against 119.0-122.6, 1030@25^2
-//    B=2 45.4 against 45.7-48.5).
+//    400 they are equal, above that four take 1-4 % less); off 4, where M is
+//    stored value by value, eight up to K = 256 (14 layers: 1 % less on average,
+//    500 -> 189@40^2 B=4 31.4 against 32.4) and four above. Channel counts off 8
+//    (M stored in pieces) have only the rules without fill: 64 rows (189@15^2
+//    B=45 28.5 against 30.0 for 96 x 128), and the 128-row tiles of K >= 512 from
+//    256 tiles and K >= 1024 below 128 (517@33^2 B=9 45.9 against 44.2 for 64
+//    rows, 1029@33^2 B=16 119.9 against 119.0-122.6, 1030@25^2 B=2 45.4 against
+//    45.7-48.5).
 // Share of a row of tiles of width t that n fills.
 static double fill(int n, int t) { return (double)n / (t * ((n + t - 1) / t)); }
 
@@ -631,7 +633,7 @@ static int wgemm_cfg(int K, int Cp, int BP) {
     if ((K >= 640 && BP >= 64) || (K >= 512 && BP >= 128) || (K >= 256 && BP >= 200) ||
         (K <= 128 && BP >= 1600))
         return narrow ? 7 : 6;
-    return grid(64, 64) >= 300 ? 1 : 4;
+    return (K % 4 == 0 ? grid(64, 64) >= 300 : K > 256) ? 1 : 4;
 }
 
 int wgemm_stream_v(int K, int Cp, int BP) {

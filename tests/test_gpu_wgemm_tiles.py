@@ -31,7 +31,8 @@ CASES = [
     (9, 72, 696, 30, "<64, 128, 2, 4, 2>"),    # BP 225, K past a tile
     (1, 24, 40, 36, "<64, 64, 2, 4, 2>"),      # BP 36, M staged
     # K % 8 != 0: M stored in pieces of four channels, or one by one (odd K)
-    (8, 66, 130, 25, "<64, 64, 2, 2, 2>"),     # BP 200
+    (8, 66, 130, 25, "<64, 64, 2, 4, 2>"),     # BP 200
+    (8, 66, 132, 25, "<64, 64, 2, 2, 2>"),     # BP 200, four channels a piece
     (5, 9, 33, 30, "<64, 64, 2, 4, 2>"),       # BP 125, one partial stage
     (9, 77, 700, 30, "<64, 128, 2, 4, 2>"),    # BP 225
     (9, 40, 517, 33, "<128, 128, 2, 4, 2>"),   # BP 324

@@ -56,6 +56,8 @@ def test_wide_layers_take_128_rows_from_256_tiles(tile):
 def test_64_row_tiles_take_four_waves_from_300_workgroups(tile):
     assert tile([(128, 128, 128), (200, 200, 144), (333, 336, 64), (576, 576, 50),
                  (64, 64, 1024)]) == [(64, 64, 8)] + [(64, 64, 4)] * 4
+    # off 4 channels: eight up to 256, four above
+    assert tile([(141, 144, 560), (333, 336, 64)]) == [(64, 64, 8), (64, 64, 4)]
 
 
 def test_wide_layers_off_64_bytes_or_small_are_not_streamed(stream_v):
