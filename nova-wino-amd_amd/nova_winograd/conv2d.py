@@ -523,8 +523,9 @@ class NovaWinogradConv2d(nn.Module):
             self._weight_version = weight._version
             # the workspace follows the layer's shape and device (and
             # _ensure_workspace's stream): new values of the same parameter (an
-            # optimizer step) keep it
-            if ref is None or ref[1][3:] != key[3:]:
+            # optimizer step) keep it, except in a graph capture, which takes
+            # its own
+            if ref is None or ref[1][3:] != key[3:] or torch.cuda.is_current_stream_capturing():
                 self._V_gemm = None
                 self._M_gemm = None
                 self._last_config = None
@@ -536,12 +537,14 @@ class NovaWinogradConv2d(nn.Module):
 
         The workspace is used on the stream it was allocated on and on no
         other, so the caching allocator may hand it on in that stream's order
-        when it is dropped. A call in a graph capture takes its own from the
-        graph's pool, and the next call outside takes another: replays write
-        to memory that no later call of the module gives up."""
-        capturing = torch.cuda.is_current_stream_capturing()
+        when it is dropped. One that a graph capture allocated is that
+        graph's alone (the next call takes another): replays write to memory
+        that no later call of the module gives up. A capture with unchanged
+        weights on the very stream of the last eager call is not looked for
+        (0.3 us a call) and records that call's workspace; on a stream of its
+        own, as ``torch.cuda.graph`` captures by itself, it has its own."""
         config = (batch, H, W, self.padding, self._handle.stream)
-        if capturing or self._last_config != config:
+        if self._last_config != config:
             self._last_config = self._state = None
             self._V_gemm = self._M_gemm = None
             nh, nw, H_out, W_out = compute_tiling(H, W, self.padding)
@@ -556,7 +559,7 @@ class NovaWinogradConv2d(nn.Module):
                 self._M_gemm = torch.empty(64, self.out_channels, BP, dtype=torch.float16,
                                            device=device)
             self._tiling = (nh, nw, H_out, W_out)
-            if not capturing:
+            if not torch.cuda.is_current_stream_capturing():
                 self._last_config = config
         return self._tiling
 
@@ -638,11 +641,7 @@ class NovaWinogradConv2d(nn.Module):
     def _remember(self, x):
         """Record what the fast path of ``forward`` checks and replays. The
         weight and bias objects are held, so their identities cannot be
-        reused by other tensors while the record exists. The fast path does
-        not look for a capture (0.3 us a call): a graph captured on the very
-        stream of the last eager call replays on that call's workspace, and
-        one captured on a stream of its own, as ``torch.cuda.graph`` does by
-        itself, on its own."""
+        reused by other tensors while the record exists."""
         hd = self._handle
         B, C, H, W = x.shape
         nh, nw, H_out, W_out = self._tiling

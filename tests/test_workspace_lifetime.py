@@ -14,16 +14,33 @@ from nova_winograd import NovaWinogradConv2d, NovaWinogradConv2dTrainable
 DEV = torch.device("cuda:0")
 
 
+class Handle:
+    """The library handle's part in it: a stream, the key of the last weights
+    and a layer that needs a workspace."""
+
+    h, key, stream = None, None, 1
+    lib = SimpleNamespace(nova_workspace_bytes=lambda h, b, H, W, pad: 1)
+
+    def set_stream(self, device):
+        pass
+
+    def set_weights(self, weight):
+        pass
+
+
 @pytest.fixture
 def module(monkeypatch):
     state = SimpleNamespace(capturing=False)
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: state.capturing)
     mod = NovaWinogradConv2d(8, 8)
-    mod._handle = SimpleNamespace(h=None, stream=1, lib=SimpleNamespace(
-        nova_workspace_bytes=lambda h, b, H, W, pad: 1))
+    mod._handle = Handle()
     mod.capture = state
 
-    def workspace(batch=2):
+    def workspace(batch=2, new_weights=False):
+        if new_weights:
+            with torch.no_grad():
+                mod.weight.add_(1.0)
+        mod._ensure_handle()
         mod._ensure_workspace(batch, 14, 14)
         assert mod._V_gemm.numel() == 64 * 8 * batch * 16 and mod._M_gemm.shape == mod._V_gemm.shape
         return mod._V_gemm, mod._M_gemm
@@ -39,27 +56,33 @@ def other(a, b):
 def test_same_stream_and_shape_keep_the_workspace(module):
     a = module.workspace()
     assert not other(a, module.workspace())
+    assert not other(a, module.workspace(new_weights=True))
     assert other(a, module.workspace(3))
 
 
-def test_another_stream_takes_its_own(module):
+@pytest.mark.parametrize("new_weights", [False, True])
+def test_another_stream_takes_its_own(module, new_weights):
     a = module.workspace()
     module._handle.stream = 2
-    b = module.workspace()
+    b = module.workspace(new_weights=new_weights)
     assert other(a, b)
     assert not other(b, module.workspace())
 
 
-def test_a_capture_takes_its_own_and_leaves_none(module):
+@pytest.mark.parametrize("new_weights", [False, True])
+def test_a_capture_takes_its_own_and_leaves_none(module, new_weights):
     a = module.workspace()
+    # on a stream of its own, or with new weights on the eager calls' stream
+    module._handle.stream = 1 if new_weights else 2
     module.capture.capturing = True
-    b = module.workspace()
+    b = module.workspace(new_weights=new_weights)
     assert other(a, b)
     module.capture.capturing = False
     c = module.workspace()  # same stream, same shape: not the graph's
     assert other(b, c)
-    module.capture.capturing = True  # another capture on that stream
-    assert other(c, module.workspace())
+    module._handle.stream = 2 if new_weights else 3
+    module.capture.capturing = True  # another capture
+    assert other(c, module.workspace(new_weights=new_weights))
 
 
 def test_a_failed_allocation_leaves_no_record(module, monkeypatch):
@@ -97,7 +120,8 @@ def step(mod, x, gy):
 
 
 @pytest.mark.gpu
-def test_captured_training_step_keeps_its_workspace():
+@pytest.mark.parametrize("same_stream", [False, True])
+def test_captured_training_step_keeps_its_workspace(same_stream):
     C, B, H = 192, 6, 20
     x = torch.randn(B, C, H, H, device=DEV).half().requires_grad_()
     gy = (0.01 * torch.randn(B, C, H, H, device=DEV)).half()
@@ -120,7 +144,7 @@ def test_captured_training_step_keeps_its_workspace():
     eager = {mod._V_gemm.data_ptr(), mod._M_gemm.data_ptr()}
     print("[workspace, captured step] capture", flush=True)
     g = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(g):
+    with torch.cuda.graph(g, stream=s if same_stream else None):
         out = step(mod, x, gy)
     captured = {mod._V_gemm.data_ptr(), mod._M_gemm.data_ptr()}
     assert not eager & captured
