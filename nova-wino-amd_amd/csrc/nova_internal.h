@@ -321,7 +321,7 @@ hipError_t launch_wgrad(const uint16_t* x, const void* dy, bool dy_f32, float* d
 // Direct form for fp16 dY (wgrad_direct.hip): nine taps as fp16 MFMA products
 // over the pixels, the operands read as they are, fp32 sums. ok is false
 // where the form does not apply (pads above 2, no images, x or dY of 2 GiB less
-// 64 KB and the two rows that dY's resource starts above it).
+// the two rows that dY's resource starts above it).
 struct WgradDirectPlan {
     int wk, wc;         // waves along output and input channels (of 8)
     int G, R, nrb;      // images and x rows per unit, row blocks per image

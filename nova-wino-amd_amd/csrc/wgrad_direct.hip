@@ -629,10 +629,11 @@ WgradDirectPlan wgrad_direct_plan(int B, int C, int K, int H, int W, int pad, in
     // pads of 3 and more have taps that reach past the halo
     if (pad > 2 || B < 1) return best;
     // 32-bit byte offsets into x and dY, and both resources, each with the
-    // rows or the chunk it starts above its tensor, end below kOob
+    // rows or the chunk it starts above its tensor, end below kOob (64 bytes
+    // for the start's offset, the last dword and a register load's reach)
     const int64_t img = 2 * std::max((int64_t)C * H * W, (int64_t)K * Ho * Wo);
     const int64_t lead = std::max<int64_t>(16, 2 * (2 - pad) * (int64_t)Wo);
-    if (B * img + lead >= ((int64_t)1 << 31) - 65536) return best;
+    if (B * img + lead > ((int64_t)1 << 31) - 64) return best;
     const int wseg = ceil_div(Wo, 8);
     double best_t = 0.0;
     for (int v = 0; v < 3; v++) {

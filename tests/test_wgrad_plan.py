@@ -57,6 +57,7 @@ def test_resources_end_below_the_offset_of_empty_lanes(plans):
 
 def test_smaller_tensors_keep_the_direct_products(plans):
     shapes = [(32, 64, 64, 56, 56, 1), (1, 1, 1, 17000, 60000, 1), (1, 1, 2, 17000, 30002, 0),
-              (1, 1, 1, 3, 3, 0), (2, 65, 40, 9, 11, 2)]
+              (1, 1, 1, 3, 3, 0), (2, 65, 40, 9, 11, 2),
+              (1, 1, 1, 1048543, 1024, 1), (1, 1, 1, 131035, 8194, 0)]  # 66 and 80 KB below 2 GiB
     assert [ok for ok, _ in plans(shapes)] == [1] * len(shapes)
     assert [ok for ok, _ in plans([(1, 4, 4, 8, 8, 3), (0, 4, 4, 8, 8, 1)])] == [0, 0]
